@@ -133,6 +133,12 @@ gdn2::Cfg make_cfg(const gdn2_desc* d) {
       if (16 * ti >= p.row0 && 16 * ti < p.row0 + p.P && 16 * tj >= p.col0 && 16 * tj < p.col0 + p.P)
         c.tile_piece[t] = pi;
     }
+    c.tile_leg[t] = 0;
+    if (c.tile_piece[t] >= 0) {
+      const gdn2::Piece& p = c.pieces.p[c.tile_piece[t]];
+      const int first = p.kind == 0 ? p.anchor : p.s0, last = p.kind == 1 ? p.s1 - 1 : first;
+      c.tile_leg[t] = p.kind | first << 8 | last << 16;
+    }
   }
   return c;
 }

@@ -423,7 +423,16 @@ __device__ __forceinline__ float4 pick4(const float4 (&x)[4], int t) {
                      sel4(x[0].z, x[1].z, x[2].z, x[3].z, t), sel4(x[0].w, x[1].w, x[2].w, x[3].w, t));
 }
 
-// STD: the pieces are the standard geometry's (bt = score_bs = 64, bs2 = 32), see std_pieces().
+// GEO: how the kernel walks the score pieces, a compile-time choice so that B4's squares, their
+// row / column tiles and the register indices that follow from them are constants:
+//   GEO_STD   the standard geometry's three squares (bt = score_bs = 64, bs2 = 32) with their
+//             anchors constant too, see std_pieces();
+//   GEO_32    the same three 32 x 32 squares (every bs2 >= 32), anchors from Cfg::tile_leg;
+//   GEO_16    the ten 16 x 16 tiles of the lower triangle (bs2 = 16), anchors from Cfg::tile_leg;
+//   GEO_LIST  the piece list walked at run time (the elementwise kernels only).
+// Walking the list at run time for bs2 = 16 or 64 as well (pieces read byte by byte from the
+// argument block, selects and branches per tile) took 159 / 99 us at B3 H5 L1472 D128 and 142 /
+// 79 us at D64, against 79 / 75 us and 60 / 55 us with constant squares.
 // EM: elementwise pieces, a compile-time choice, so that the other kernels carry no trace of
 // the elementwise loops (whose live ranges otherwise push registers into scratch):
 //   EM_NONE  every piece on MFMA;
@@ -431,10 +440,11 @@ __device__ __forceinline__ float4 pick4(const float4 (&x)[4], int t) {
 //   EM_MIX   pieces narrower than a 16 x 16 tile (bs2 = 8): every piece elementwise, with its
 //            legs (or, with the lean diagonal, the diagonal blocks exactly).
 enum { EM_NONE = 0, EM_LEAN = 1, EM_MIX = 2 };
-template <int D, int B3, bool STD, int EM>
+enum { GEO_STD = 0, GEO_32 = 1, GEO_16 = 2, GEO_LIST = 3 };
+template <int D, int B3, int GEO, int EM>
 __global__ __launch_bounds__(512) void bwd_wy_kernel(BwdWyArgs a) {
   constexpr bool ELEM = EM != EM_NONE;
-  static_assert(!(STD && ELEM), "the standard piece list is the BTL one");
+  static_assert((GEO == GEO_LIST) == ELEM, "the elementwise kernels walk the piece list");
   using Lay = BwdWyLayout<D>;
   using St = Strip<D>;
   constexpr int LD = Lay::LD, LT = Lay::LT, NT = 512, NW = 8, NTW = St::NTW, NKB = D / 16;
@@ -866,9 +876,10 @@ __global__ __launch_bounds__(512) void bwd_wy_kernel(BwdWyArgs a) {
     ar = a.anc[(size_t)chunk * 2 * D + dcol];
     az = a.anc[(size_t)chunk * 2 * D + D + dcol];
   }
-  // One piece of the two-level score factorisation; with the standard geometry the three
-  // pieces are compile-time constants, so every branch and index below folds away.
-  auto b4_piece = [&](const Piece pc) __attribute__((always_inline)) {
+  // One piece of the two-level score factorisation.  The square (row0, col0, P) is a compile-time
+  // constant except with GEO_LIST, so the branches and indices below fold away; row_leg(i) /
+  // col_leg(j) are its legs at this lane's column.
+  auto b4_square = [&](const Piece pc, auto row_leg, auto col_leg) __attribute__((always_inline)) {
     const int nb = pc.P / 16, tr0 = pc.row0 / 16, tc0 = pc.col0 / 16;
     // legs at this lane's positions; qt = q ra, bkt = (b k) ra over the piece rows,
     // kt = k cb over the piece columns (k blocks of 16)
@@ -879,8 +890,8 @@ __global__ __launch_bounds__(512) void bwd_wy_kernel(BwdWyArgs a) {
       float rv[4], cv[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        rv[e] = piece_row_leg(pc, sG, LD, 16 * ti + 4 * g + e, dcol, ar, az);
-        cv[e] = piece_col_leg(pc, sG, LD, 16 * tj + 4 * g + e, dcol, ar, az);
+        rv[e] = row_leg(16 * ti + 4 * g + e);
+        cv[e] = col_leg(16 * tj + 4 * g + e);
       }
       ra[kb] = make_float4(rv[0], rv[1], rv[2], rv[3]);
       cbl[kb] = make_float4(cv[0], cv[1], cv[2], cv[3]);
@@ -963,11 +974,38 @@ __global__ __launch_bounds__(512) void bwd_wy_kernel(BwdWyArgs a) {
       }
     }
   };
-  if constexpr (STD) {
+  auto b4_piece = [&](const Piece pc) __attribute__((always_inline)) {
+    b4_square(
+        pc, [&](int i) { return piece_row_leg(pc, sG, LD, i, dcol, ar, az); },
+        [&](int j) { return piece_col_leg(pc, sG, LD, j, dcol, ar, az); });
+  };
+  // a square whose anchors come from the packed entry of its corner tile: the legs of leg_row /
+  // leg_col with the kind folded into an offset and a bound (no branch between the MFMA chains)
+  auto b4_anchored = [&](const Piece sq) __attribute__((always_inline)) {
+    const int32_t tl = cf.tile_leg[4 * (sq.row0 / 16) + sq.col0 / 16];
+    const int kind = tl & 0xff;
+    const float ga = kind == 2 ? ar : sG[((tl >> 8) & 0xff) * LD + dcol];
+    const float gz = kind == 2 ? az : sG[((tl >> 16) & 0xff) * LD + dcol];
+    const float half = kind == 0 ? 0.f : 0.5f * (ga - gz);
+    const float top = kind == 0 ? 0.f : __builtin_inff();
+    b4_square(
+        sq, [&](int i) { return fast_exp(__builtin_elementwise_minimum((sG[i * LD + dcol] - ga) + half, top)); },
+        [&](int j) { return fast_exp(__builtin_elementwise_minimum((ga - sG[j * LD + dcol]) - half, top)); });
+  };
+  if constexpr (GEO == GEO_STD) {
     constexpr Piece P0{0, 0, 32, 1, 0, 0, 32, 0}, P1{32, 32, 32, 1, 32, 32, 64, 0}, P2{32, 0, 32, 0, 32, 0, 0, 0};
     b4_piece(P0);
     b4_piece(P1);
     b4_piece(P2);
+  } else if constexpr (GEO == GEO_32) {
+    b4_anchored(Piece{0, 0, 32, 0, 0, 0, 0, 0});
+    b4_anchored(Piece{32, 32, 32, 0, 0, 0, 0, 0});
+    b4_anchored(Piece{32, 0, 32, 0, 0, 0, 0, 0});
+  } else if constexpr (GEO == GEO_16) {
+#pragma unroll
+    for (int ti = 0; ti < 4; ++ti)
+#pragma unroll
+      for (int tj = 0; tj <= ti; ++tj) b4_anchored(Piece{(int8_t)(16 * ti), (int8_t)(16 * tj), 16, 0, 0, 0, 0, 0});
   } else {
     for (int pi = 0; pi < cf.pieces.n; ++pi) {
       const Piece pc = load_piece(cf.pieces.p[pi]);
@@ -1323,6 +1361,8 @@ hipError_t launch_bwd_wy(int D, const BwdWyArgs& a, hipStream_t s) {
   // elementwise pieces: pieces of side 8 (every piece has side min(bs2, 32)), or the lean diagonal
   const bool mix = a.cfg.pieces.p[0].P < 16, elem = mix || a.cfg.diag == DIAG_LEAN;
   const bool std_geom = !elem && std_pieces(a.cfg.pieces);
+  const int side = a.cfg.pieces.p[0].P;      // 8, 16 or 32: min(bs2, 32), and bs2 >= 8 is a power of two
+  if (side != 8 && side != 16 && side != 32) return hipErrorInvalidValue;
   // kind-2 pieces on the factorised path read the anchor buffer
   if (!elem && a.cfg.pieces.p[0].kind == 2 && !a.anc) return hipErrorInvalidValue;
   // D = 128 BTL kernels are persistent: one workgroup per CU (their LDS admits no second).
@@ -1333,15 +1373,17 @@ hipError_t launch_bwd_wy(int D, const BwdWyArgs& a, hipStream_t s) {
     constexpr int M = decltype(m)::value;
     const dim3 grid(a.n_chunks), block(512);
     if (D == 128) {
-      if (mix) hipLaunchKernelGGL((bwd_wy_kernel<128, M, false, EM_MIX>), grid, block, 0, s, a);
-      else if (elem) hipLaunchKernelGGL((bwd_wy_kernel<128, M, false, EM_LEAN>), grid, block, 0, s, a);
-      else if (std_geom) hipLaunchKernelGGL((bwd_wy_kernel<128, M, true, EM_NONE>), pgrid, block, 0, s, a);
-      else hipLaunchKernelGGL((bwd_wy_kernel<128, M, false, EM_NONE>), pgrid, block, 0, s, a);
+      if (mix) hipLaunchKernelGGL((bwd_wy_kernel<128, M, GEO_LIST, EM_MIX>), grid, block, 0, s, a);
+      else if (elem) hipLaunchKernelGGL((bwd_wy_kernel<128, M, GEO_LIST, EM_LEAN>), grid, block, 0, s, a);
+      else if (std_geom) hipLaunchKernelGGL((bwd_wy_kernel<128, M, GEO_STD, EM_NONE>), pgrid, block, 0, s, a);
+      else if (side == 32) hipLaunchKernelGGL((bwd_wy_kernel<128, M, GEO_32, EM_NONE>), pgrid, block, 0, s, a);
+      else hipLaunchKernelGGL((bwd_wy_kernel<128, M, GEO_16, EM_NONE>), pgrid, block, 0, s, a);
     } else {
-      if (mix) hipLaunchKernelGGL((bwd_wy_kernel<64, M, false, EM_MIX>), grid, block, 0, s, a);
-      else if (elem) hipLaunchKernelGGL((bwd_wy_kernel<64, M, false, EM_LEAN>), grid, block, 0, s, a);
-      else if (std_geom) hipLaunchKernelGGL((bwd_wy_kernel<64, M, true, EM_NONE>), grid, block, 0, s, a);
-      else hipLaunchKernelGGL((bwd_wy_kernel<64, M, false, EM_NONE>), grid, block, 0, s, a);
+      if (mix) hipLaunchKernelGGL((bwd_wy_kernel<64, M, GEO_LIST, EM_MIX>), grid, block, 0, s, a);
+      else if (elem) hipLaunchKernelGGL((bwd_wy_kernel<64, M, GEO_LIST, EM_LEAN>), grid, block, 0, s, a);
+      else if (std_geom) hipLaunchKernelGGL((bwd_wy_kernel<64, M, GEO_STD, EM_NONE>), grid, block, 0, s, a);
+      else if (side == 32) hipLaunchKernelGGL((bwd_wy_kernel<64, M, GEO_32, EM_NONE>), grid, block, 0, s, a);
+      else hipLaunchKernelGGL((bwd_wy_kernel<64, M, GEO_16, EM_NONE>), grid, block, 0, s, a);
     }
     return 0;
   });

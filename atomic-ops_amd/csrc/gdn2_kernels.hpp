@@ -66,6 +66,9 @@ struct Cfg {
   // byte load, and a vector load of kernel arguments would make its wait cover every memory
   // operation in flight).
   int32_t tile_piece[16];
+  // the legs of that piece, packed for the backward: kind | anchor row << 8 | last row << 16 (kind
+  // 0: the anchor row; kind 1: the block's first and last rows; kind 2: rows in the anchor buffer)
+  int32_t tile_leg[16];
 };
 
 // Piece i of a piece list held in the kernel arguments, read as two scalar dwords (i wave-uniform)

@@ -81,11 +81,22 @@ def lib():
         L.gdn2_debug_gemm.argtypes = [_c_int, _vp, _vp, _vp, _c_int, _c_int, _c_int, _vp]
         L.gdn2_debug_stream.argtypes = [_c_int, _vp, _vp, _c_size, _vp]
         L.gdn2_debug_mfma.argtypes = [_c_int, _c_int, _vp, _vp]
+        L.gdn2_lm_premix_workspace_bytes.argtypes = [_c_int] * 4
+        L.gdn2_lm_premix_workspace_bytes.restype = _c_size
+        L.gdn2_lm_premix_fwd.argtypes = [_vp, _vp]
+        L.gdn2_lm_premix_bwd.argtypes = [_vp, P(_vp)] + [_vp] * 5
+        L.gdn2_lm_rms_workspace_bytes.argtypes = [_c_int, _c_int]
+        L.gdn2_lm_rms_workspace_bytes.restype = _c_size
+        L.gdn2_lm_rms_fwd.argtypes = [_vp, _vp]
+        L.gdn2_lm_rms_bwd.argtypes = [_vp, _vp]
+        L.gdn2_lm_swiglu.argtypes = [_vp, _vp, _vp, _c_int, _c_int, _vp]
+        L.gdn2_lm_columns.argtypes = [_c_int, P(_vp), P(_c_int), _c_int, _vp, _c_int, _c_int, _vp]
         L.gdn2_prof_begin.argtypes = [_c_int]
         L.gdn2_prof_end.argtypes = [P(_c_dbl), P(_c_int)]
         for fn in ("gdn2_residual_layout", "gdn2_fwd", "gdn2_fwd_bf16", "gdn2_fwd_noalloc", "gdn2_fwd_reset",
                    "gdn2_decode", "gdn2_bwd", "gdn2_wy_stage", "gdn2_scores", "gdn2_debug_gemm", "gdn2_debug_stream",
-                   "gdn2_debug_mfma", "gdn2_prof_begin", "gdn2_prof_end"):
+                   "gdn2_debug_mfma", "gdn2_lm_premix_fwd", "gdn2_lm_premix_bwd", "gdn2_lm_rms_fwd", "gdn2_lm_rms_bwd",
+                   "gdn2_lm_swiglu", "gdn2_lm_columns", "gdn2_prof_begin", "gdn2_prof_end"):
             getattr(L, fn).restype = _c_int
         if L.gdn2_abi_version() != ABI_VERSION:
             raise Gdn2Error("libgdn2_hip.so ABI version mismatch")

@@ -18,7 +18,9 @@ uniform tokens in [0, vocab).  Matmuls run in fp32 (the reference sets
 ``jax_default_matmul_precision='highest'``).
 
 This module is the operator's caller, written with torch (no flax / optax in this image); the
-operator itself is ``make_blr_trainable`` on the HIP kernels.
+operator itself is ``make_blr_trainable`` on the HIP kernels.  On the GPU in float32 a block's
+element-wise chains run as HIP kernels too (``lm_kernels``); the module code below is the same
+computation in torch operations, for every other device, dtype and mixer.
 """
 from __future__ import annotations
 
@@ -29,6 +31,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
+from . import lm_kernels
 from .config import make_cfg
 from .pipeline import make_blr_trainable
 
@@ -75,6 +78,7 @@ def blhd_kernel(cfg, d_head):
         o, _ = fn(*(sw(x) for x in (q, k, v, w, b, g)))
         return o.transpose(1, 2)
 
+    run.head_major = fn       # the operator itself, for callers whose tensors are head-major already
     return run
 
 
@@ -105,7 +109,7 @@ class RMSNorm(nn.Module):
         self.eps = eps
 
     def forward(self, x):
-        return x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + self.eps) * self.scale
+        return lm_kernels.rms_ref(x, self.scale, self.eps)
 
 
 class CausalDepthwiseConv(nn.Module):
@@ -120,11 +124,7 @@ class CausalDepthwiseConv(nn.Module):
     def forward(self, x):                      # (B, L, C)
         # K shifted multiply-adds on the (B, L, C) layout: element-wise work that streams x
         # K times, instead of a grouped convolution with one group per channel
-        K = self.k
-        y = torch.addcmul(self.bias, x, self.weight[:, K - 1])
-        for s in range(1, K):
-            y = torch.addcmul(y, F.pad(x[:, :-s], (0, 0, s, 0)), self.weight[:, K - 1 - s])
-        return y
+        return lm_kernels.conv_ref(x, self.weight, self.bias)
 
 
 class GDN2Block(nn.Module):
@@ -145,6 +145,8 @@ class GDN2Block(nn.Module):
         self.down_proj = Dense(cfg.mlp_mult * d, d, False)
 
     def forward(self, x):
+        if lm_kernels.usable(self, x, Dense, CausalDepthwiseConv, RMSNorm):
+            return lm_kernels.block_forward(self, x)
         cfg = self.cfg
         B, L, _ = x.shape
         H, D = cfg.n_heads, cfg.d_head
@@ -156,9 +158,7 @@ class GDN2Block(nn.Module):
         k = k * torch.rsqrt((k * k).sum(-1, keepdim=True) + eps)
         beta = torch.sigmoid(self.erase_gate(x)).reshape(B, L, H, D)
         wg = torch.sigmoid(self.write_gate(x)).reshape(B, L, H, D)
-        ldh = -torch.exp(self.decay_a.clamp(-20, 20)) * F.softplus(self.decay_proj(x))
-        ld = torch.nan_to_num(ldh, nan=0.0, posinf=0.0, neginf=-20.0)
-        g = (-ld.abs().clamp(max=cfg.g_max)).unsqueeze(-1).expand(B, L, H, D)
+        g = lm_kernels.decay_ref(self.decay_proj(x), self.decay_a, cfg.g_max).unsqueeze(-1).expand(B, L, H, D)
         o = self.kernel_fn(q, k, v, wg, beta, g).reshape(B, L, H * D)
         og = self.out_gate(x)
         x = x + self.out_proj(self.mixer_out_norm(o) * F.silu(og))
@@ -178,6 +178,9 @@ class LM(nn.Module):
         x = self.embed[ids]
         for blk in self.blocks:
             x = blk(x)
+        if (len(self.blocks) and getattr(self.blocks[-1].kernel_fn, "head_major", None) is not None
+                and lm_kernels.norm_usable(self.final_norm, x, RMSNorm)):
+            return lm_kernels.rms_norm(self.final_norm, x) @ self.embed.t()
         return self.final_norm(x) @ self.embed.t()
 
 

@@ -1,0 +1,363 @@
+"""The language-model block of ``e2e_lm`` on the HIP passes of ``csrc/gdn2_lm.hip``.
+
+``block_forward`` computes what ``GDN2Block.forward`` computes, with the element-wise chains
+between the matrix products in one kernel each and the products that share an input as one GEMM:
+
+* ``_PreMix``   x -> one GEMM with [Wq | Wk | Wv | We | Ww | Wo | Wd] -> q, k, v, w, b, g head-major,
+  the layout the operator reads, and the output gate's logits;
+* ``_PostMix``  the operator's o -> RMS norm, SiLU gate, output projection, residual;
+* ``_Mlp``      RMS norm, gate / up as one GEMM, SiLU(gate) * up, down projection, residual.
+
+Each is one autograd node whose backward runs the matching backward kernels.  A backward that is
+itself to be differentiated (``create_graph``) recomputes the step from ``_premix_ref`` /
+``_postmix_ref`` / ``_mlp_ref``, the same in torch operations.
+
+``usable`` says where this path stands in for the module's own forward: float32 on the GPU, the
+block's own submodule types without hooks, the HIP operator as the mixer.  Everywhere else (the CPU,
+other dtypes, autocast, hooked or replaced submodules, another mixer) the module forward runs.
+"""
+from __future__ import annotations
+
+import ctypes
+
+import torch
+import torch.nn.functional as F
+
+from . import _lib
+
+_i32, _f32c, _vp = ctypes.c_int32, ctypes.c_float, ctypes.c_void_p
+_EPS = 1e-6
+_MAX_C = 1024           # widest row of the RMS kernels
+
+
+class _PremixArgs(ctypes.Structure):
+    _fields_ = [("B", _i32), ("L", _i32), ("H", _i32), ("D", _i32), ("ldy", _i32), ("g_max", _f32c), ("y", _vp),
+                ("conv_w", _vp * 3), ("conv_b", _vp * 3), ("gate_b", _vp * 2), ("decay_b", _vp), ("decay_a", _vp),
+                ("out", _vp * 6), ("og", _vp)]
+
+
+class _RmsArgs(ctypes.Structure):
+    _fields_ = [("rows", _i32), ("C", _i32), ("L", _i32), ("D", _i32)] + [
+        (n, _vp) for n in ("x", "gate", "scale", "dy", "res", "y", "dx", "dgate", "part", "dscale")]
+
+
+def _addr(t):
+    return None if t is None else t.data_ptr()
+
+
+def _dense(t):
+    """t as the kernels read it: contiguous, 16-byte aligned."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+def _call(name, dev, *args):
+    fn = getattr(_lib.lib(), name)
+    with torch.cuda.device(dev):
+        _lib.check(fn(*args, _lib.stream_handle(dev)), name)
+
+
+def _rms(x, scale, gate=None, heads=None):
+    """RMS norm of the rows of x (N, C), or of the head-major o with heads = (L, D) and a gate."""
+    rows, C = (x.shape[0], x.shape[1]) if gate is None else (gate.shape[0], gate.shape[1])
+    y = torch.empty((rows, C), dtype=torch.float32, device=x.device)
+    L, D = heads or (0, 0)
+    a = _RmsArgs(rows, C, L, D, _addr(x), _addr(gate), _addr(scale), None, None, _addr(y), None, None, None, None)
+    _call("gdn2_lm_rms_fwd", x.device, ctypes.byref(a))
+    return y
+
+
+def _rms_bwd(x, scale, dy, gate=None, heads=None, res=None):
+    rows, C = dy.shape
+    dev = x.device
+    dx, dscale = torch.empty_like(x), torch.empty_like(scale)
+    dgate = None if gate is None else torch.empty_like(gate)
+    part = torch.empty(_lib.lib().gdn2_lm_rms_workspace_bytes(rows, C) // 4, dtype=torch.float32, device=dev)
+    L, D = heads or (0, 0)
+    a = _RmsArgs(rows, C, L, D, _addr(x), _addr(gate), _addr(scale), _addr(dy), _addr(res), None, _addr(dx),
+                 _addr(dgate), _addr(part), _addr(dscale))
+    _call("gdn2_lm_rms_bwd", dev, ctypes.byref(a))
+    return dx, dscale, dgate
+
+
+def _swiglu(gu, d_act=None):
+    rows, M2 = gu.shape
+    out = torch.empty((rows, M2 // 2 if d_act is None else M2), dtype=torch.float32, device=gu.device)
+    _call("gdn2_lm_swiglu", gu.device, _addr(gu), _addr(d_act), _addr(out), rows, M2 // 2)
+    return out
+
+
+def _columns(split, parts, wide):
+    n = len(parts)
+    ptrs = (_vp * n)(*(t.data_ptr() for t in parts))
+    widths = (_i32 * n)(*(t.shape[1] for t in parts))
+    _call("gdn2_lm_columns", wide.device, int(split), ptrs, widths, n, _addr(wide), wide.shape[0], wide.shape[1])
+
+
+def _gather(parts, ld):
+    """The matrices side by side, zero-padded to ld columns."""
+    wide = torch.empty((parts[0].shape[0], ld), dtype=torch.float32, device=parts[0].device)
+    _columns(0, parts, wide)
+    return wide
+
+
+def _scatter(wide, like):
+    """wide back into contiguous matrices of the shapes of ``like``."""
+    flat = torch.empty(sum(t.numel() for t in like), dtype=torch.float32, device=wide.device)
+    out, o = [], 0
+    for t in like:
+        out.append(flat[o:o + t.numel()].view(t.shape))
+        o += t.numel()
+    _columns(1, out, wide)
+    return out
+
+
+def _vjp_through(ref, inputs, needs, grads):
+    """Gradients of ref(*inputs) for a backward that is itself differentiated."""
+    with torch.enable_grad():
+        outs = ref(*inputs)
+        outs = outs if isinstance(outs, tuple) else (outs,)
+        pairs = [(o, g) for o, g in zip(outs, grads) if g is not None and o.requires_grad]
+        wrt = [x for x, n in zip(inputs, needs) if n]
+        got = iter(torch.autograd.grad([o for o, _ in pairs], wrt, [g for _, g in pairs], create_graph=True,
+                                       allow_unused=True))
+    return tuple(next(got) if n else None for n in needs)
+
+
+# ------------------------------------------------------------------------------------------
+# the steps in torch operations
+# ------------------------------------------------------------------------------------------
+
+def conv_ref(x, weight, bias):
+    """Causal depthwise convolution of (B, L, C): K shifted multiply-adds."""
+    K = weight.shape[1]
+    y = torch.addcmul(bias, x, weight[:, K - 1])
+    for s in range(1, K):
+        y = torch.addcmul(y, F.pad(x[:, :-s], (0, 0, s, 0)), weight[:, K - 1 - s])
+    return y
+
+
+def rms_ref(x, scale, eps=_EPS):
+    return x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + eps) * scale
+
+
+def decay_ref(logits, decay_a, g_max):
+    """Per-head log-decay (B, L, H) of the decay logits."""
+    ldh = -torch.exp(decay_a.clamp(-20, 20)) * F.softplus(logits)
+    ld = torch.nan_to_num(ldh, nan=0.0, posinf=0.0, neginf=-20.0)
+    return -ld.abs().clamp(max=g_max)
+
+
+def _premix_ref(H, D, g_max):
+    def ref(x, wq, wk, wv, we, ww, wo, wd, cqw, cqb, ckw, ckb, cvw, cvb, be, bw, bd, da):
+        B, L, _ = x.shape
+        heads = lambda y: y.reshape(B, L, H, D).transpose(1, 2)  # noqa: E731
+        q, k, v = (heads(F.silu(conv_ref(x @ w, cw, cb)))
+                   for w, cw, cb in ((wq, cqw, cqb), (wk, ckw, ckb), (wv, cvw, cvb)))
+        q, k = (y * torch.rsqrt((y * y).sum(-1, keepdim=True) + _EPS) for y in (q, k))
+        b, w = heads(torch.sigmoid(x @ we + be)), heads(torch.sigmoid(x @ ww + bw))
+        g = decay_ref(x @ wd + bd, da, g_max).transpose(1, 2).unsqueeze(-1).expand(B, H, L, D)
+        return q, k, v.clamp(-50.0, 50.0), w, b, g, (x @ wo).reshape(B * L, H * D)
+    return ref
+
+
+def _postmix_ref(o, og, x, scale, wo):
+    B, H, L, D = o.shape
+    z = rms_ref(o.transpose(1, 2).reshape(B * L, H * D), scale) * F.silu(og)
+    return x + (z @ wo).reshape(x.shape)
+
+
+def _mlp_ref(x, scale, wg, wu, wd):
+    h = rms_ref(x, scale)
+    return x + (F.silu(h @ wg) * (h @ wu)) @ wd
+
+
+# ------------------------------------------------------------------------------------------
+# the autograd nodes
+# ------------------------------------------------------------------------------------------
+
+class _PreMix(torch.autograd.Function):
+    """(x, Wq, Wk, Wv, We, Ww, Wo, Wd, conv taps and biases of q, k, v, be, bw, bd, decay_a) ->
+    q, k, v, w, b, g (B, H, L, D), output-gate logits (B L, C)."""
+
+    @staticmethod
+    def forward(ctx, H, D, g_max, x, *ps):
+        B, L, d = x.shape
+        C, dev = H * D, x.device
+        ws = ps[:7]
+        ldy = -(-(6 * C + H) // 64) * 64
+        wide = _gather(ws, ldy)
+        y = x.reshape(B * L, d) @ wide
+        outs = [torch.empty((B, H, L, D), dtype=torch.float32, device=dev) for _ in range(6)]
+        og = torch.empty((B * L, C), dtype=torch.float32, device=dev)
+        a = _PreMix._args(H, D, g_max, x, ps, y, outs, og)
+        _call("gdn2_lm_premix_fwd", dev, ctypes.byref(a))
+        ctx.dims = (H, D, g_max)
+        ctx.save_for_backward(x, *ps, wide, y, *outs, og)
+        return (*outs, og)
+
+    @staticmethod
+    def _args(H, D, g_max, x, ps, y, outs, og):
+        cqw, cqb, ckw, ckb, cvw, cvb, be, bw, bd, da = (t.data_ptr() for t in ps[7:])
+        return _PremixArgs(x.shape[0], x.shape[1], H, D, y.shape[1], float(g_max), y.data_ptr(), (_vp * 3)(cqw, ckw, cvw),
+                           (_vp * 3)(cqb, ckb, cvb), (_vp * 2)(be, bw), bd, da, (_vp * 6)(*(t.data_ptr() for t in outs)),
+                           og.data_ptr())
+
+    @staticmethod
+    def backward(ctx, *gs):
+        H, D, g_max = ctx.dims
+        saved = ctx.saved_tensors
+        x, ps, wide, y, outs, og = saved[0], saved[1:18], saved[18], saved[19], saved[20:26], saved[26]
+        if torch.is_grad_enabled():
+            return (None, None, None) + _vjp_through(_premix_ref(H, D, g_max), (x,) + ps, ctx.needs_input_grad[3:], gs)
+        B, L, d = x.shape
+        C, dev, N = H * D, x.device, x.shape[0] * x.shape[1]
+        like = list(outs) + [og]
+        ds = [torch.zeros_like(t) if g is None else _dense(g) for g, t in zip(gs, like)]
+        dy = torch.empty_like(y)
+        dparam = torch.empty(17 * C + 2 * H, dtype=torch.float32, device=dev)
+        ws = torch.empty(_lib.lib().gdn2_lm_premix_workspace_bytes(B, L, H, D), dtype=torch.uint8, device=dev)
+        a = _PreMix._args(H, D, g_max, x, ps, y, outs, og)
+        _call("gdn2_lm_premix_bwd", dev, ctypes.byref(a), (_vp * 6)(*(t.data_ptr() for t in ds[:6])), _addr(ds[6]),
+              _addr(dy), _addr(dparam), _addr(ws))
+        need = ctx.needs_input_grad[3:]
+        dx = (dy @ wide.t()).reshape(B, L, d) if need[0] else None
+        dws = _scatter(x.reshape(N, d).t() @ dy, ps[:7]) if any(need[1:8]) else [None] * 7
+        dps, o = [], 0
+        for t in ps[7:]:
+            dps.append(dparam[o:o + t.numel()].view(t.shape))
+            o += t.numel()
+        return (None, None, None) + tuple(g if n else None for g, n in zip([dx, *dws, *dps], need))
+
+
+class _PostMix(torch.autograd.Function):
+    """(o (B, H, L, D), output-gate logits, x, norm scale, Wout) -> x + (rms(o) scale silu(og)) Wout."""
+
+    @staticmethod
+    def forward(ctx, o, og, x, scale, wo):
+        B, H, L, D = o.shape
+        z = _rms(o, scale, og, (L, D))
+        ctx.save_for_backward(o, og, x, scale, wo, z)
+        return torch.addmm(x.reshape(B * L, -1), z, wo).reshape(x.shape)
+
+    @staticmethod
+    def backward(ctx, dy):
+        o, og, x, scale, wo, z = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return _vjp_through(_postmix_ref, (o, og, x, scale, wo), ctx.needs_input_grad, (dy,))
+        need = ctx.needs_input_grad
+        B, H, L, D = o.shape
+        d2 = dy.reshape(B * L, -1)
+        do = dog = dscale = None
+        if need[0] or need[1] or need[3]:
+            do, dscale, dog = _rms_bwd(o, scale, d2 @ wo.t(), og, (L, D))
+        dwo = z.t() @ d2 if need[4] else None
+        return tuple(g if n else None for g, n in zip((do, dog, dy, dscale, dwo), need))
+
+
+class _Mlp(torch.autograd.Function):
+    """(x, norm scale, Wgate, Wup, Wdown) -> x + (silu(h Wgate) (h Wup)) Wdown, h = rms(x) scale."""
+
+    @staticmethod
+    def forward(ctx, x, scale, wg, wu, wd):
+        x2 = x.reshape(-1, x.shape[-1])
+        h = _rms(x2, scale)
+        wide = _gather((wg, wu), 2 * wg.shape[1])
+        gu = h @ wide
+        act = _swiglu(gu)
+        ctx.save_for_backward(x, scale, wg, wu, wd, h, wide, gu, act)
+        return torch.addmm(x2, act, wd).reshape(x.shape)
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, scale, wg, wu, wd, h, wide, gu, act = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return _vjp_through(_mlp_ref, (x, scale, wg, wu, wd), ctx.needs_input_grad, (dy,))
+        need = ctx.needs_input_grad
+        d2 = _dense(dy.reshape(-1, dy.shape[-1]))
+        dgu = _swiglu(gu, d2 @ wd.t())
+        dwd = act.t() @ d2 if need[4] else None
+        dwg, dwu = _scatter(h.t() @ dgu, (wg, wu)) if need[2] or need[3] else (None, None)
+        dx, dscale, _ = _rms_bwd(x.reshape(d2.shape), scale, dgu @ wide.t(), res=d2)
+        return tuple(g if n else None for g, n in zip((dx.reshape(x.shape), dscale, dwg, dwu, dwd), need))
+
+
+class _RmsNorm(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, scale):
+        ctx.save_for_backward(x, scale)
+        return _rms(x.reshape(-1, x.shape[-1]), scale).reshape(x.shape)
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, scale = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return _vjp_through(rms_ref, (x, scale), ctx.needs_input_grad, (dy,))
+        d2 = _dense(dy.reshape(-1, dy.shape[-1]))
+        dx, dscale, _ = _rms_bwd(x.reshape(d2.shape), scale, d2)
+        return dx.reshape(x.shape), dscale
+
+
+# ------------------------------------------------------------------------------------------
+# the block
+# ------------------------------------------------------------------------------------------
+
+_HOOKS = ("_forward_hooks", "_forward_pre_hooks", "_backward_hooks", "_backward_pre_hooks")
+_DENSE = ("q_proj", "k_proj", "v_proj", "erase_gate", "write_gate", "out_gate", "decay_proj", "out_proj", "gate_proj",
+          "up_proj", "down_proj")
+_CONV = ("q_conv", "k_conv", "v_conv")
+_NORM = ("mixer_out_norm", "mlp_norm")
+_BIASED = ("erase_gate", "write_gate", "decay_proj")
+
+
+def _ready(t, dev):
+    return (t.device == dev and t.dtype == torch.float32 and t.is_contiguous() and t.data_ptr() % 16 == 0
+            and t.numel() > 0)
+
+
+def _plain(m, cls):
+    return type(m) is cls and not any(getattr(m, h) for h in _HOOKS)
+
+
+def _usable_input(x):
+    return (x.is_cuda and type(x) in (torch.Tensor, torch.nn.Parameter) and _ready(x, x.device)
+            and x.shape[-1] % 4 == 0 and x.shape[-1] <= _MAX_C and not torch.is_autocast_enabled("cuda")
+            and not torch.nn.modules.module._has_any_global_hook())
+
+
+def usable(block, x, dense, conv, norm):
+    """Whether block_forward stands for block.forward(x); dense, conv, norm: the module types that
+    the block is built of."""
+    fn = getattr(block.kernel_fn, "head_major", None)
+    c = block.cfg
+    if fn is None or not (x.dim() == 3 and _usable_input(x)):
+        return False
+    if c.d_head not in (64, 128) or c.d_conv != 4 or c.proj_dim > _MAX_C or (c.mlp_mult * c.d_model) % 4:
+        return False
+    mods = block._modules
+    if not (all(_plain(mods[n], dense) for n in _DENSE) and all(_plain(mods[n], conv) for n in _CONV)
+            and all(_plain(mods[n], norm) and mods[n].eps == _EPS for n in _NORM)):
+        return False
+    if any((mods[n].bias is None) == (n in _BIASED) for n in _DENSE):
+        return False
+    return all(type(p) is torch.nn.Parameter and _ready(p, x.device) for p in block.parameters())
+
+
+def norm_usable(module, x, norm):
+    return (_plain(module, norm) and module.eps == _EPS and _usable_input(x) and type(module.scale) is torch.nn.Parameter
+            and _ready(module.scale, x.device))
+
+
+def rms_norm(module, x):
+    return _RmsNorm.apply(x, module.scale)
+
+
+def block_forward(m, x):
+    c = m.cfg
+    *ops, og = _PreMix.apply(
+        c.n_heads, c.d_head, c.g_max, x, m.q_proj.weight, m.k_proj.weight, m.v_proj.weight, m.erase_gate.weight,
+        m.write_gate.weight, m.out_gate.weight, m.decay_proj.weight, m.q_conv.weight, m.q_conv.bias, m.k_conv.weight,
+        m.k_conv.bias, m.v_conv.weight, m.v_conv.bias, m.erase_gate.bias, m.write_gate.bias, m.decay_proj.bias, m.decay_a)
+    o, _ = m.kernel_fn.head_major(*ops)
+    x = _PostMix.apply(o, og, x, m.mixer_out_norm.scale, m.out_proj.weight)
+    return _Mlp.apply(x, m.mlp_norm.scale, m.gate_proj.weight, m.up_proj.weight, m.down_proj.weight)

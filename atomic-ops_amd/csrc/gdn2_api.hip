@@ -1,5 +1,6 @@
 // C ABI of the GDN-2 library: descriptor validation, residual / workspace layout, kernel
 // sequencing per segment, and optional per-kernel HIP-event timing.
+#include <initializer_list>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -565,6 +566,142 @@ int gdn2_debug_gemm(int mode, const float* A, const float* B, float* C, int M, i
   hipError_t e = gdn2::launch_gemm_probe(mode, A, B, C, M, N, K, reinterpret_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "gemm probe launch");
   return GDN2_OK;
+}
+
+namespace {
+int lm_shape(int B, int L, int H, int D) {
+  if (B < 1 || L < 1 || H < 1) return fail(GDN2_ERR_INVALID, "non-positive shape");
+  if (D != 64 && D != 128) return fail(GDN2_ERR_UNSUPPORTED, "D in {64, 128} only");
+  if ((int64_t)B * L > (int64_t(1) << 27) || H > 4096 || (int64_t)B * H * ((L + 127) / 128) > 0x7fffffff)
+    return fail(GDN2_ERR_UNSUPPORTED, "shape too large");
+  return GDN2_OK;
+}
+bool aligned16(std::initializer_list<const void*> ps) {
+  uintptr_t x = 0;
+  for (const void* p : ps) x |= reinterpret_cast<uintptr_t>(p);
+  return (x & 15) == 0;
+}
+int lm_premix_args(const gdn2_lm_premix* p, gdn2::LmPremixArgs* a) {
+  if (!p) return fail(GDN2_ERR_INVALID, "null argument block");
+  const int st = lm_shape(p->B, p->L, p->H, p->D);
+  if (st) return st;
+  if (p->ldy < 6 * p->H * p->D + p->H || p->ldy % 4) return fail(GDN2_ERR_INVALID, "ldy too small or not a multiple of 4");
+  a->y = p->y;
+  bool ok = p->y && p->decay_b && p->decay_a && p->og && aligned16({p->y, p->og});
+  for (int i = 0; i < 3; ++i) {
+    a->cw[i] = p->conv_w[i];
+    a->cb[i] = p->conv_b[i];
+    ok = ok && p->conv_w[i] && p->conv_b[i] && aligned16({p->conv_w[i], p->conv_b[i]});
+  }
+  for (int i = 0; i < 2; ++i) {
+    a->gb[i] = p->gate_b[i];
+    ok = ok && p->gate_b[i] && aligned16({p->gate_b[i]});
+  }
+  for (int i = 0; i < 6; ++i) {
+    a->out[i] = p->out[i];
+    ok = ok && p->out[i] && aligned16({p->out[i]});
+  }
+  if (!ok) return fail(GDN2_ERR_INVALID, "null or misaligned pointer (16 bytes)");
+  a->decay_b = p->decay_b;
+  a->decay_a = p->decay_a;
+  a->og = p->og;
+  a->B = p->B; a->L = p->L; a->H = p->H; a->ldy = p->ldy;
+  a->g_max = p->g_max;
+  return GDN2_OK;
+}
+int lm_rms_args(const gdn2_lm_rms* p, gdn2::LmRmsArgs* a) {
+  if (!p) return fail(GDN2_ERR_INVALID, "null argument block");
+  if (p->rows < 1 || p->C < 4 || p->C % 4 || p->C > 1024 || p->rows > (1 << 27))
+    return fail(GDN2_ERR_UNSUPPORTED, "rms rows of 4 .. 1024 floats, a multiple of 4");
+  if (p->gate && (p->L < 1 || p->rows % p->L || p->D < 4 || p->D % 4 || p->C % p->D))
+    return fail(GDN2_ERR_INVALID, "gated rms: rows = B L, C = H D, D a multiple of 4");
+  if (!p->x || !p->scale || !aligned16({p->x, p->gate, p->scale, p->dy, p->res, p->y, p->dx, p->dgate, p->part}))
+    return fail(GDN2_ERR_INVALID, "null or misaligned pointer (16 bytes)");
+  a->x = p->x; a->gate = p->gate; a->scale = p->scale; a->dy = p->dy; a->res = p->res;
+  a->y = p->y; a->dx = p->dx; a->dgate = p->dgate; a->part = p->part; a->dscale = p->dscale;
+  a->rows = p->rows; a->C = p->C; a->L = p->L; a->D = p->D;
+  a->inv_c = 1.f / (float)p->C;
+  return GDN2_OK;
+}
+int lm_done(hipError_t e, const char* what) { return e == hipSuccess ? GDN2_OK : hip_fail(e, what); }
+}  // namespace
+
+size_t gdn2_lm_premix_workspace_bytes(int B, int L, int H, int D) {
+  if (lm_shape(B, L, H, D)) return 0;
+  return (size_t)gdn2::lm_premix_rows(B, L) * (17 * (size_t)H * D + 2 * H) * 4;
+}
+
+int gdn2_lm_premix_fwd(const gdn2_lm_premix* p, void* stream) {
+  gdn2::LmPremixArgs a{};
+  const int st = lm_premix_args(p, &a);
+  if (st) return st;
+  return lm_done(gdn2::launch_lm_premix_fwd(p->D, a, reinterpret_cast<hipStream_t>(stream)), "lm premix launch");
+}
+
+int gdn2_lm_premix_bwd(const gdn2_lm_premix* p, const float* const d_out[6], const float* d_og, float* dy,
+                       float* dparam, void* workspace, void* stream) {
+  gdn2::LmPremixBwdArgs a{};
+  const int st = lm_premix_args(p, &a.f);
+  if (st) return st;
+  if (!d_out || !d_og || !dy || !dparam || !workspace || !aligned16({d_og, dy}))
+    return fail(GDN2_ERR_INVALID, "null or misaligned pointer (16 bytes)");
+  for (int i = 0; i < 6; ++i) {
+    if (!d_out[i] || !aligned16({d_out[i]})) return fail(GDN2_ERR_INVALID, "null or misaligned pointer (16 bytes)");
+    a.d[i] = d_out[i];
+  }
+  a.dog = d_og;
+  a.dy = dy;
+  a.part = static_cast<float*>(workspace);
+  a.dparam = dparam;
+  return lm_done(gdn2::launch_lm_premix_bwd(p->D, a, reinterpret_cast<hipStream_t>(stream)), "lm premix backward launch");
+}
+
+size_t gdn2_lm_rms_workspace_bytes(int rows, int C) {
+  return rows < 1 || C < 1 ? 0 : (size_t)gdn2::lm_rms_parts(rows) * C * 4;
+}
+
+int gdn2_lm_rms_fwd(const gdn2_lm_rms* p, void* stream) {
+  gdn2::LmRmsArgs a{};
+  const int st = lm_rms_args(p, &a);
+  if (st) return st;
+  if (!a.y) return fail(GDN2_ERR_INVALID, "null tensor pointer");
+  return lm_done(gdn2::launch_lm_rms_fwd(a, reinterpret_cast<hipStream_t>(stream)), "lm rms launch");
+}
+
+int gdn2_lm_rms_bwd(const gdn2_lm_rms* p, void* stream) {
+  gdn2::LmRmsArgs a{};
+  const int st = lm_rms_args(p, &a);
+  if (st) return st;
+  if (!a.dy || !a.dx || !a.part || !a.dscale || (a.gate && !a.dgate)) return fail(GDN2_ERR_INVALID, "null tensor pointer");
+  return lm_done(gdn2::launch_lm_rms_bwd(a, reinterpret_cast<hipStream_t>(stream)), "lm rms backward launch");
+}
+
+int gdn2_lm_swiglu(const float* gu, const float* d_act, float* out, int rows, int M, void* stream) {
+  if (rows < 1 || M < 4 || M % 4 || (int64_t)rows * (M / 4) > (int64_t(1) << 38))
+    return fail(GDN2_ERR_INVALID, "swiglu rows of a multiple of 4 floats");
+  if (!gu || !out || !aligned16({gu, d_act, out})) return fail(GDN2_ERR_INVALID, "null or misaligned pointer (16 bytes)");
+  return lm_done(gdn2::launch_lm_swiglu(gu, d_act, out, rows, M, reinterpret_cast<hipStream_t>(stream)), "lm swiglu launch");
+}
+
+int gdn2_lm_columns(int split, float* const parts[], const int32_t widths[], int n, float* wide, int rows, int ld,
+                    void* stream) {
+  if (n < 1 || n > gdn2::LM_MAX_PARTS || rows < 1 || rows > 65535 || ld < 1) return fail(GDN2_ERR_INVALID, "bad shape");
+  if (!parts || !widths || !wide) return fail(GDN2_ERR_INVALID, "null pointer");
+  gdn2::LmColumnsArgs a{};
+  int64_t c = 0;
+  for (int j = 0; j < n; ++j) {
+    if (!parts[j] || widths[j] < 1) return fail(GDN2_ERR_INVALID, "null part or non-positive width");
+    a.part[j] = parts[j];
+    a.width[j] = widths[j];
+    a.start[j] = (int)c;
+    c += widths[j];
+    if (c > ld) return fail(GDN2_ERR_INVALID, "parts wider than ld");
+  }
+  a.wide = wide;
+  a.n = n;
+  a.rows = rows;
+  a.ld = ld;
+  return lm_done(gdn2::launch_lm_columns(a, split != 0, reinterpret_cast<hipStream_t>(stream)), "lm columns launch");
 }
 
 int gdn2_debug_stream(int mode, const void* src, void* dst, size_t bytes, void* stream) {

@@ -286,6 +286,49 @@ hipError_t launch_stream_probe(int mode, const void* src, void* dst, size_t n4, 
 // (512 iters).
 hipError_t launch_mfma_probe(int blocks, int iters, float* out, hipStream_t s);
 
+// ---- the language-model block's passes around the operator (gdn2_lm.hip) -----------------------
+// Rows y of the wide projection (row stride ldy): columns [q | k | v | erase | write | output gate]
+// of C = H D each, then H decay logits, then padding.  cw / cb: the depthwise convolutions' taps
+// (C, 4) and biases (q, k, v); gb: the erase and write gates' biases; out: q, k, v, w, b, g
+// head-major (B, H, L, D); og: the output gate's logits (B L, C).
+struct LmPremixArgs {
+  const float* y;
+  const float *cw[3], *cb[3], *gb[2], *decay_b, *decay_a;
+  float* out[6];
+  float* og;
+  int B, L, H, ldy;
+  float g_max;
+};
+// d: the gradients of out, dog of og; dy like y; part: lm_premix_rows(B, L) rows of
+// 17 C + 2 H floats (workspace), dparam: their sum.
+struct LmPremixBwdArgs {
+  LmPremixArgs f;
+  const float *d[6], *dog;
+  float *dy, *part, *dparam;
+};
+// RMS norm of rows of C floats; gate != null: x is head-major (B, H, L, D), y times SiLU(gate).
+struct LmRmsArgs {
+  const float *x, *gate, *scale, *dy, *res;    // dy, res: backward
+  float *y, *dx, *dgate, *part, *dscale;       // y: forward; the others: backward
+  int rows, C, L, D;
+  float inv_c;
+};
+constexpr int LM_MAX_PARTS = 8;
+struct LmColumnsArgs {
+  float* part[LM_MAX_PARTS];
+  int width[LM_MAX_PARTS], start[LM_MAX_PARTS];
+  float* wide;
+  int n, rows, ld;
+};
+int lm_premix_rows(int B, int L);
+int lm_rms_parts(int rows);
+hipError_t launch_lm_premix_fwd(int D, const LmPremixArgs& a, hipStream_t s);
+hipError_t launch_lm_premix_bwd(int D, const LmPremixBwdArgs& a, hipStream_t s);
+hipError_t launch_lm_rms_fwd(const LmRmsArgs& a, hipStream_t s);
+hipError_t launch_lm_rms_bwd(const LmRmsArgs& a, hipStream_t s);
+hipError_t launch_lm_swiglu(const float* gu, const float* dact, float* out, int rows, int M, hipStream_t s);
+hipError_t launch_lm_columns(const LmColumnsArgs& a, bool split, hipStream_t s);
+
 // Linear work index of this workgroup such that consecutive indices (workgroups of one
 // (batch, head), which read the same chunk operands) land on the same XCD (blockIdx % 8 picks
 // the XCD) and are served from that XCD's L2.  Identity unless nblk % 8 == 0.

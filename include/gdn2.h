@@ -202,6 +202,57 @@ int gdn2_wy_stage(const gdn2_desc* d, const float* q, const float* k, const floa
 int gdn2_scores(const gdn2_desc* d, const float* q, const float* k, const float* b, const float* gc,
                 float* aqk, float* akk, void* stream);
 
+/* ---- the language-model block around the operator ------------------------------------------
+ * The element-wise and row-wise passes of the reference's benchmark LM block (GDN2Block; notebook
+ * benchmarks/notebooks/all-paths-speed.ipynb, cell 2) between its matrix products, all float32
+ * with 16-byte aligned tensors. */
+
+/* Rows y (B*L, ldy) of the products of x with [Wq | Wk | Wv | We | Ww | Wo | Wd]: six blocks of
+ * C = H*D columns, H decay logits, padding.  conv_w (C,4) and conv_b (C) of q, k, v; gate_b (C) of
+ * the erase and write gates; decay_b, decay_a (H).  out: q, k, v, w, b, g as (B,H,L,D):
+ *   q, k = l2norm_D(silu(conv(y))) (eps 1e-6), v = clip(silu(conv(y)), +-50),
+ *   b = sigmoid(ye + bias), w = sigmoid(yw + bias),
+ *   g = -min(|nan_to_num(-exp(clip(decay_a, +-20)) softplus(yd + decay_b))|, g_max);
+ * conv: out[t] = sum_j y[t-3+j] w[j] + bias, zero before t = 0.  og (B*L, C): a copy of yo. */
+typedef struct gdn2_lm_premix {
+  int32_t B, L, H, D;     /* D in {64, 128} */
+  int32_t ldy;            /* >= 6*H*D + H, a multiple of 4 */
+  float g_max;
+  const float* y;
+  const float *conv_w[3], *conv_b[3], *gate_b[2], *decay_b, *decay_a;
+  float *out[6], *og;
+} gdn2_lm_premix;
+int gdn2_lm_premix_fwd(const gdn2_lm_premix* p, void* stream);
+/* Its VJP: d_out (six tensors like out) and d_og -> dy (every column, padding zero) and dparam,
+ * 17 C + 2 H floats: for q, k, v the taps (C,4) then the biases (C); the erase and write biases;
+ * decay_b; decay_a.  p->out holds the forward's outputs. */
+size_t gdn2_lm_premix_workspace_bytes(int B, int L, int H, int D);
+int gdn2_lm_premix_bwd(const gdn2_lm_premix* p, const float* const d_out[6], const float* d_og, float* dy,
+                       float* dparam, void* workspace, void* stream);
+
+/* y = x rsqrt(mean(x^2) + 1e-6) scale over rows of C floats (C <= 1024, a multiple of 4).  With a
+ * gate (rows, C), x is the operator's output (B,H,L,D), rows = B*L, C = H*D, and y is further
+ * multiplied by silu(gate).  Backward: dy (and, without a gate, optionally res, added to dx) ->
+ * dx (like x), dgate, dscale (C); part: gdn2_lm_rms_workspace_bytes. */
+typedef struct gdn2_lm_rms {
+  int32_t rows, C, L, D;  /* L, D: with a gate only */
+  const float *x, *gate, *scale, *dy, *res;
+  float *y, *dx, *dgate, *part, *dscale;
+} gdn2_lm_rms;
+size_t gdn2_lm_rms_workspace_bytes(int rows, int C);
+int gdn2_lm_rms_fwd(const gdn2_lm_rms* p, void* stream);
+int gdn2_lm_rms_bwd(const gdn2_lm_rms* p, void* stream);
+
+/* gu (rows, 2M) = [gate | up].  d_act NULL: out (rows, M) = silu(gate) up; else out (rows, 2M) =
+ * the gradient of gu for d_act (rows, M). */
+int gdn2_lm_swiglu(const float* gu, const float* d_act, float* out, int rows, int M, void* stream);
+
+/* n <= 8 matrices parts[j] (rows, widths[j]) and one (rows, ld) matrix that holds them side by side:
+ * split 0 gathers them (columns past the last are zeroed), split 1 scatters it back.
+ * rows <= 65535. */
+int gdn2_lm_columns(int split, float* const parts[], const int32_t widths[], int n, float* wide, int rows,
+                    int ld, void* stream);
+
 /* Diagnostics: C[M,N] = A[M,K] B[K,N] (row-major float32) through the kernels' MFMA tile
  * routine in the given dot mode.  M, N <= 64, K <= 128, all multiples of 16. */
 int gdn2_debug_gemm(int mode, const float* A, const float* B, float* C, int M, int N, int K,

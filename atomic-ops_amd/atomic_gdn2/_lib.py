@@ -75,6 +75,7 @@ def lib():
         L.gdn2_fwd_noalloc.argtypes = [P(Gdn2Desc)] + [_vp] * 10
         L.gdn2_fwd_reset.argtypes = [P(Gdn2Desc), _c_int] + [_vp] * 12
         L.gdn2_decode.argtypes = [P(Gdn2DecodeDesc)] + [_vp] * 13
+        L.gdn2_decode_flags.argtypes = [P(Gdn2DecodeDesc), _c_int] + [_vp] * 13
         L.gdn2_bwd.argtypes = [P(Gdn2Desc)] + [_vp] * 18
         L.gdn2_wy_stage.argtypes = [P(Gdn2Desc)] + [_vp] * 15
         L.gdn2_scores.argtypes = [P(Gdn2Desc)] + [_vp] * 7
@@ -94,7 +95,7 @@ def lib():
         L.gdn2_prof_begin.argtypes = [_c_int]
         L.gdn2_prof_end.argtypes = [P(_c_dbl), P(_c_int)]
         for fn in ("gdn2_residual_layout", "gdn2_fwd", "gdn2_fwd_bf16", "gdn2_fwd_noalloc", "gdn2_fwd_reset",
-                   "gdn2_decode", "gdn2_bwd", "gdn2_wy_stage", "gdn2_scores", "gdn2_debug_gemm", "gdn2_debug_stream",
+                   "gdn2_decode", "gdn2_decode_flags", "gdn2_bwd", "gdn2_wy_stage", "gdn2_scores", "gdn2_debug_gemm", "gdn2_debug_stream",
                    "gdn2_debug_mfma", "gdn2_lm_premix_fwd", "gdn2_lm_premix_bwd", "gdn2_lm_rms_fwd", "gdn2_lm_rms_bwd",
                    "gdn2_lm_swiglu", "gdn2_lm_columns", "gdn2_prof_begin", "gdn2_prof_end"):
             getattr(L, fn).restype = _c_int
@@ -102,6 +103,25 @@ def lib():
             raise Gdn2Error("libgdn2_hip.so ABI version mismatch")
         _LIB = L
     return _LIB
+
+
+_BIND = None
+_BIND_ABI = ("gdn2_residual_layout", "gdn2_fwd_workspace_bytes", "gdn2_bwd_workspace_bytes", "gdn2_fwd", "gdn2_fwd_bf16",
+             "gdn2_bwd", "gdn2_decode_flags", "gdn2_last_error")
+
+
+def bind():
+    """The native call path (csrc/bind.cpp) on the loaded library; raise loudly if it is not there."""
+    global _BIND
+    if _BIND is None:
+        L = lib()
+        try:
+            from . import _bind
+        except ImportError as e:
+            raise Gdn2Error(f"atomic_gdn2/_bind.so is not built ({e}); run `python atomic-ops_amd/build_lib.py`") from e
+        _bind.bind(*(ctypes.cast(getattr(L, n), _vp).value for n in _BIND_ABI))
+        _BIND = _bind
+    return _BIND
 
 
 def check(status: int, what: str):

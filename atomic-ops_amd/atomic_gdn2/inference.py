@@ -137,6 +137,14 @@ def decode_step(q=None, k=None, v=None, w=None, b=None, g=None, state=None,
         q, k, v, w, b, g = inputs.as_tuple()
     if q is None or state is None:
         raise ValueError("pass either inputs=LayerInputs(...) or q,k,v,w,b,g,state")
+    if isinstance(q, torch.Tensor) and q.is_cuda and state_dtype in _STATE_DTYPES and type(scale) in (int, float) \
+            and (stability_tau is None or type(stability_tau) in (int, float)) and type(fuse_prologue) is bool:
+        # plain calls (csrc/bind.cpp) go native; None = not one, and what follows handles it
+        out = _lib.bind().decode(q, k, v, w, b, g, state, float(scale), reset, _STATE_DTYPES[state_dtype] == 1,
+                                 None if stability_tau is None else float(stability_tau), fuse_prologue,
+                                 a_log if fuse_prologue else None, dt_bias if fuse_prologue else None)
+        if out is not None:
+            return out
     bsz, H, D = q.shape
     if not isinstance(scale, (int, float)) or isinstance(scale, torch.Tensor):
         raise ValueError(

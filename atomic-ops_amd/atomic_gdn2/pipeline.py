@@ -14,7 +14,9 @@ Drop-in for the reference's ``atomic_gdn2/pipeline.py:17-66``:
   (``gdn2_desc.seq_ld``): no slice copies, gradient scatters or concatenation.
 
 Every call goes to the HIP kernels in ``libgdn2_hip.so``; there is no other backend.  Tensors
-must live on a ROCm device.
+must live on a ROCm device.  Plain calls (float32, or bfloat16 without gradients, on one device) take
+the native call path (``csrc/bind.cpp``), which does what the Python below does; this file handles
+every other dtype and kind of call, and all errors.
 """
 from __future__ import annotations
 
@@ -94,6 +96,7 @@ def make_blr_trainable(cfg, scale, state_ckpt=None):
     ckpt = DEFAULT_STATE_CKPT if state_ckpt is None else int(state_ckpt)
     if ckpt < 0:
         raise ValueError(f"state_ckpt={ckpt} must be >= 0")
+    native = None        # this configuration on the native call path, made at the first call
 
     class _Sequence(torch.autograd.Function):
         """The whole call as one autograd node.  Forward and backward run the reference's
@@ -188,6 +191,15 @@ def make_blr_trainable(cfg, scale, state_ckpt=None):
 
     def call(q, k, v, w, b, g, h0=None):
         """q..g: (B,H,L,D), L % bt == 0. Returns (o (B,H,L,D) f32, h_final (B,H,D,D) f32)."""
+        nonlocal native
+        if isinstance(q, torch.Tensor) and q.is_cuda:
+            # plain calls (csrc/bind.cpp) go native; None = not one, and what follows handles it
+            if native is None:
+                native = _lib.bind().op(bytes(_lib.make_desc(cfg, 0, 0, 0, 0, scale, state_ckpt=ckpt)),
+                                        cfg.max_chunks_per_call * cfg.bt)
+            out = _lib.bind().sequence(native, q, k, v, w, b, g, h0)
+            if out is not None:
+                return out
         _check_inputs((q, k, v, w, b, g), "qkvwbg")
         bsz, H, L, D = q.shape
         if L % cfg.bt:

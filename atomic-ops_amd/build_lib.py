@@ -1,4 +1,5 @@
-"""Build ``libgdn2_hip.so`` in-tree with hipcc for gfx950.
+"""Build ``libgdn2_hip.so`` in-tree with hipcc for gfx950, and the native call path ``_bind.so``
+(host C++ against this torch) with g++.
 
 Usage: ``python atomic-ops_amd/build_lib.py`` (also called by ``__graft_entry__.build()``).
 Each ``csrc/*.hip`` translation unit is compiled to an object in ``_build/`` in parallel,
@@ -55,12 +56,37 @@ def _compile(src: Path, verbose: bool) -> Path:
     return obj
 
 
+def _build_bind(verbose: bool) -> Path:
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    out = HERE / "atomic_gdn2" / "_bind.so"
+    tmp = BUILD / "_bind.so.tmp"
+    lib = Path(torch.__file__).resolve().parent / "lib"
+    rocm = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
+    incs = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"], str(rocm / "include")]
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-w",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-I{i}" for i in incs), str(CSRC / "bind.cpp"), "-o", str(tmp), f"-L{lib}", f"-Wl,-rpath,{lib}",
+           "-Wl,--no-as-needed", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on bind.cpp:\n{r.stdout}\n{r.stderr}")
+    os.replace(tmp, out)
+    return out
+
+
 def build(verbose: bool = False) -> Path:
     BUILD.mkdir(exist_ok=True)
     OUT.parent.mkdir(parents=True, exist_ok=True)
     srcs = sorted(CSRC.glob("*.hip"))
-    with cf.ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
+    with cf.ThreadPoolExecutor(max_workers=8) as ex:
+        bind = ex.submit(_build_bind, verbose)
         objs = list(ex.map(lambda s: _compile(s, verbose), srcs))
+        bind.result()
     tmp = OUT.with_suffix(".so.tmp")
     cmd = [_hipcc(), "-shared", "-fPIC", f"--offload-arch={ARCH}", *map(str, objs), "-o", str(tmp)]
     if verbose:

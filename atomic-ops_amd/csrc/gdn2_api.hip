@@ -368,6 +368,13 @@ int gdn2_fwd_bf16(const gdn2_desc* d, const uint16_t* q, const uint16_t* k, cons
 int gdn2_decode(const gdn2_decode_desc* d, const void* q, const void* k, const void* v, const void* w,
                 const void* b, const void* g, const float* a_log, const float* dt_bias, const uint8_t* reset,
                 const void* state_in, void* o, void* state_out, void* stream) {
+  return gdn2_decode_flags(d, GDN2_FLAG_BYTE, q, k, v, w, b, g, a_log, dt_bias, reset, state_in, o, state_out, stream);
+}
+
+int gdn2_decode_flags(const gdn2_decode_desc* d, int flag_type, const void* q, const void* k, const void* v,
+                      const void* w, const void* b, const void* g, const float* a_log, const float* dt_bias,
+                      const void* reset, const void* state_in, void* o, void* state_out, void* stream) {
+  if (flag_type < GDN2_FLAG_BYTE || flag_type > GDN2_FLAG_INT64) return fail(GDN2_ERR_INVALID, "unknown flag type");
   if (!d) return fail(GDN2_ERR_INVALID, "null descriptor");
   if (d->B < 1 || d->H < 1 || d->n_tok < 1) return fail(GDN2_ERR_INVALID, "non-positive shape");
   if ((int64_t)d->B * d->H > (int64_t(1) << 22)) return fail(GDN2_ERR_UNSUPPORTED, "B*H above 4194304");
@@ -379,7 +386,7 @@ int gdn2_decode(const gdn2_decode_desc* d, const void* q, const void* k, const v
   if (d->fuse_prologue && (!a_log || !dt_bias)) return fail(GDN2_ERR_INVALID, "fuse_prologue needs a_log and dt_bias");
   gdn2::DecodeArgs a{};
   a.q = q; a.k = k; a.v = v; a.w = w; a.b = b; a.g = g;
-  a.a_log = a_log; a.dt_bias = dt_bias; a.reset = reset; a.state_in = state_in;
+  a.a_log = a_log; a.dt_bias = dt_bias; a.reset = reset; a.flag_type = flag_type; a.state_in = state_in;
   a.o = o; a.state_out = state_out;
   a.H = d->H; a.n_tok = d->n_tok; a.seq_ld = d->seq_ld;
   a.in_bf16 = d->in_dtype; a.out_bf16 = d->out_dtype; a.state_bf16 = d->state_dtype;

@@ -64,6 +64,13 @@ __device__ __forceinline__ float4 clean4(const float4& x, bool bf) {
   return y;
 }
 
+// A reset flag in the caller's own type (gdn2_decode_flags): no cast launches around a one-token call
+__device__ __forceinline__ bool flag_set(const void* p, int type, size_t i) {
+  if (type == 1) return static_cast<const int32_t*>(p)[i] > 0;
+  if (type == 2) return (int32_t)static_cast<const int64_t*>(p)[i] > 0;
+  return static_cast<const uint8_t*>(p)[i] != 0;
+}
+
 template <int D, int CW, bool CAP, bool IBF, bool SBF>
 __global__ __launch_bounds__(CW / 4 * 16) void decode_kernel(DecodeArgs a) {
   constexpr int KG = 16, NQ = CW / 4, NT = NQ * KG, KPK = D / KG, NS = D / CW, NWV = (NT + WAVE - 1) / WAVE;
@@ -88,7 +95,7 @@ __global__ __launch_bounds__(CW / 4 * 16) void decode_kernel(DecodeArgs a) {
     // this thread's columns of w and v, issued with the key vectors' loads (one round trip)
     float4 wj = ld_quad<IBF>(a.w, io + j0);
     const float4 vj = ld_quad<IBF>(a.v, io + j0);
-    if (a.reset && a.reset[(size_t)bi * a.n_tok + t]) {
+    if (a.reset && flag_set(a.reset, a.flag_type, (size_t)bi * a.n_tok + t)) {
 #pragma unroll
       for (int i = 0; i < KPK; ++i) h[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     }

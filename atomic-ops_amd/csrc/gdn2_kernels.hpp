@@ -222,16 +222,17 @@ struct BwdWyArgs {
 // Token recurrence for serving (gdn2_decode.hip): n_tok tokens per (batch, head) in order.
 // q..g (and o) at ((b H + h) seq_ld + t) D + d, fp32 or bfloat16 bits (in_bf16 / out_bf16);
 // state_in / state_out (B, H, D, D) row-major (key, value) in the state dtype (state_bf16),
-// state_in null = zero state, state_out may equal state_in; reset: null or B x n_tok bytes,
-// nonzero = zero state entering that token of batch row b; fuse: q, k l2-normalised, b, w
+// state_in null = zero state, state_out may equal state_in; reset: null or B x n_tok flags of
+// flag_type (gdn2_decode_flags), set = zero state entering that token of batch row b; fuse: q, k l2-normalised, b, w
 // sigmoid, g = -exp(a_log[h]) softplus(g + dt_bias[d]) in the kernel; cap: per-head Frobenius
 // cap tau on the state.
 struct DecodeArgs {
   const void *q, *k, *v, *w, *b, *g;
   const float *a_log, *dt_bias;
-  const uint8_t* reset;
+  const void* reset;
   const void* state_in;
   void *o, *state_out;
+  int flag_type;
   int H, n_tok, seq_ld;
   int in_bf16, out_bf16, state_bf16, fuse, cap;
   float scale, tau;

@@ -167,6 +167,17 @@ int gdn2_decode(const gdn2_decode_desc* d, const void* q, const void* k, const v
                 const float* dt_bias, const uint8_t* reset, const void* state_in, void* o,
                 void* state_out, void* stream);
 
+/* gdn2_decode with the reset flags in the caller's own type: GDN2_FLAG_BYTE as gdn2_decode (set
+ * when nonzero); GDN2_FLAG_INT32 set when > 0; GDN2_FLAG_INT64 set when > 0 after a cast to
+ * int32.  B*n_tok flags, or NULL. */
+#define GDN2_FLAG_BYTE 0
+#define GDN2_FLAG_INT32 1
+#define GDN2_FLAG_INT64 2
+int gdn2_decode_flags(const gdn2_decode_desc* d, int flag_type, const void* q, const void* k,
+                      const void* v, const void* w, const void* b, const void* g,
+                      const float* a_log, const float* dt_bias, const void* reset,
+                      const void* state_in, void* o, void* state_out, void* stream);
+
 /* Forward of one segment without a residual, like gdn2_fwd(d, ..., residual = NULL, ...), with
  * the workspace in a fixed 64 MiB (67108864-byte) device array inside the library instead of
  * a caller buffer.  No counterpart in the reference: it is for callers that cannot allocate

@@ -70,6 +70,8 @@ def lib():
         L.gdn2_fwd_workspace_bytes.restype = _c_size
         L.gdn2_bwd_workspace_bytes.argtypes = [P(Gdn2Desc)]
         L.gdn2_bwd_workspace_bytes.restype = _c_size
+        L.gdn2_default_state_ckpt.argtypes = [P(Gdn2Desc)]
+        L.gdn2_default_state_ckpt.restype = _c_int
         L.gdn2_fwd.argtypes = [P(Gdn2Desc)] + [_vp] * 12
         L.gdn2_fwd_bf16.argtypes = [P(Gdn2Desc)] + [_vp] * 12
         L.gdn2_fwd_noalloc.argtypes = [P(Gdn2Desc)] + [_vp] * 10
@@ -107,7 +109,7 @@ def lib():
 
 _BIND = None
 _BIND_ABI = ("gdn2_residual_layout", "gdn2_fwd_workspace_bytes", "gdn2_bwd_workspace_bytes", "gdn2_fwd", "gdn2_fwd_bf16",
-             "gdn2_bwd", "gdn2_decode_flags", "gdn2_last_error")
+             "gdn2_bwd", "gdn2_decode_flags", "gdn2_default_state_ckpt", "gdn2_last_error")
 
 
 def bind():
@@ -138,6 +140,14 @@ def make_desc(cfg, B, H, L, D, scale, seq_ld=0, state_ckpt=0) -> Gdn2Desc:
                     DIAG_IDS[cfg.diag], DOT_IDS[cfg.dot_mode], DOT_IDS[cfg.solve_dot_mode],
                     DOT_IDS[cfg.b3_dot_mode], int(seq_ld), int(state_ckpt), float(scale),
                     float(cfg.wy_eps), float(cfg.clip), float(cfg.diff_clip))
+
+
+def training_desc(cfg, B, H, L, D, scale, seq_ld, state_ckpt) -> Gdn2Desc:
+    """make_desc with the library's checkpoint interval for the shape when state_ckpt is None."""
+    d = make_desc(cfg, B, H, L, D, scale, seq_ld=seq_ld, state_ckpt=state_ckpt or 0)
+    if state_ckpt is None:
+        d.state_ckpt = lib().gdn2_default_state_ckpt(ctypes.byref(d))
+    return d
 
 
 def residual_layout(desc: Gdn2Desc):

@@ -41,9 +41,11 @@ def kernels_support(bt, wy_eps):
 # state entering the first chunk of each checkpoint block (blocks of K chunks; up to two chunks
 # left over become blocks of their own) and the backward recomputes the others inside its state
 # reductions; 0 keeps every chunk's (as the reference's residual does, pipeline.py:25).
-# K = 3 keeps 12 of every 32 states at or slightly below the stored form's time (MI355X, B4 H6
-# D128, rounds interleaved: 0.5024 vs 0.5043 ms at L = 2048, 0.9726 vs 0.9776 ms at L = 4096);
-# K = 4 keeps a quarter for 2 % more time, K = 8 an eighth for 8 %.
+# The choice for state_ckpt=None is the library's (gdn2_default_state_ckpt): K = 3 for launches that
+# fill the chip, keeping 12 of every 32 states at or slightly below the stored form's time (MI355X,
+# B4 H6 D128: 0.4545 vs 0.4603 ms at L = 2048, 0.8807 vs 0.8945 ms at L = 4096; K = 4 keeps a
+# quarter for 3 % more time), and shorter blocks for smaller ones, whose backward is bound by a
+# block's length.
 DEFAULT_STATE_CKPT = 3
 
 
@@ -93,8 +95,8 @@ def make_blr_trainable(cfg, scale, state_ckpt=None):
     DEFAULT_STATE_CKPT; it changes memory and time, not results (the recomputed states equal
     the stored ones bit for bit)."""
     scale = float(scale)
-    ckpt = DEFAULT_STATE_CKPT if state_ckpt is None else int(state_ckpt)
-    if ckpt < 0:
+    ckpt = None if state_ckpt is None else int(state_ckpt)
+    if ckpt is not None and ckpt < 0:
         raise ValueError(f"state_ckpt={ckpt} must be >= 0")
     native = None        # this configuration on the native call path, made at the first call
 
@@ -121,7 +123,7 @@ def make_blr_trainable(cfg, scale, state_ckpt=None):
             with torch.cuda.device(dev):
                 stream = _lib.stream_handle(dev)
                 for t0, t1 in _segments(L, cfg):
-                    desc = _lib.make_desc(cfg, B, H, t1 - t0, D, scale, seq_ld=L, state_ckpt=ckpt)
+                    desc = _lib.training_desc(cfg, B, H, t1 - t0, D, scale, L, ckpt)
                     _, tot = _lib.residual_layout(desc)      # validates the descriptor
                     res = torch.empty(tot, dtype=torch.uint8, device=dev) if need_res else None
                     ws = torch.empty(L_.gdn2_fwd_workspace_bytes(ctypes.byref(desc), int(need_res)),
@@ -195,7 +197,7 @@ def make_blr_trainable(cfg, scale, state_ckpt=None):
         if isinstance(q, torch.Tensor) and q.is_cuda:
             # plain calls (csrc/bind.cpp) go native; None = not one, and what follows handles it
             if native is None:
-                native = _lib.bind().op(bytes(_lib.make_desc(cfg, 0, 0, 0, 0, scale, state_ckpt=ckpt)),
+                native = _lib.bind().op(bytes(_lib.make_desc(cfg, 0, 0, 0, 0, scale, state_ckpt=-1 if ckpt is None else ckpt)),
                                         cfg.max_chunks_per_call * cfg.bt)
             out = _lib.bind().sequence(native, q, k, v, w, b, g, h0)
             if out is not None:

@@ -39,6 +39,7 @@ struct Abi {
   decltype(&gdn2_fwd_bf16) fwd_bf16;
   decltype(&gdn2_bwd) bwd;
   decltype(&gdn2_decode_flags) decode;
+  decltype(&gdn2_default_state_ckpt) default_ckpt;
   decltype(&gdn2_last_error) last_error;
 } abi{};
 
@@ -76,6 +77,12 @@ struct Op {
   gdn2_desc base;
   int64_t segment;     // tokens per segment (max_chunks_per_call * bt)
 
+  // base.state_ckpt < 0: the library's choice for the shape
+  gdn2_desc training_desc(int64_t B, int64_t H, int64_t L, int64_t D, int64_t seq_ld) const {
+    gdn2_desc d = desc(B, H, L, D, seq_ld, base.state_ckpt);
+    if (d.state_ckpt < 0) d.state_ckpt = abi.default_ckpt(&d);
+    return d;
+  }
   gdn2_desc desc(int64_t B, int64_t H, int64_t L, int64_t D, int64_t seq_ld, int ckpt) const {
     gdn2_desc d = base;
     d.B = (int32_t)B;
@@ -103,7 +110,7 @@ struct Sequence : torch::autograd::Function<Sequence> {
     Tensor o = empty_on(q, {B, H, L, D}, at::kFloat);
     variable_list saved(xs, xs + 6);
     for (int64_t t0 = 0; t0 < L; t0 += op->segment) {
-      const gdn2_desc d = op->desc(B, H, std::min(L - t0, op->segment), D, L, op->base.state_ckpt);
+      const gdn2_desc d = op->training_desc(B, H, std::min(L - t0, op->segment), D, L);
       size_t off[GDN2_RES_COUNT], total = 0;
       if (abi.residual_layout(&d, off, &total)) throw Refused();
       Tensor res = empty_on(q, {(int64_t)total}, at::kByte);
@@ -137,7 +144,7 @@ struct Sequence : torch::autograd::Function<Sequence> {
     const int64_t n_seg = (L + op->segment - 1) / op->segment;
     for (int64_t s = n_seg - 1; s >= 0; --s) {
       const int64_t t0 = s * op->segment, x = t0 * D;
-      const gdn2_desc d = op->desc(B, H, std::min(L - t0, op->segment), D, L, op->base.state_ckpt);
+      const gdn2_desc d = op->training_desc(B, H, std::min(L - t0, op->segment), D, L);
       Tensor ws = empty_on(xs[0], {(int64_t)abi.bwd_ws(&d)}, at::kByte);
       Tensor dh0 = empty_on(xs[0], {B, H, D, D}, at::kFloat);
       const int st = abi.bwd(&d, f32_at(xs[0], x), f32_at(xs[1], x), f32_at(xs[2], x), f32_at(xs[3], x),

@@ -262,6 +262,20 @@ size_t gdn2_fwd_workspace_bytes(const gdn2_desc* d, int with_residual) {
   return n;
 }
 
+// A checkpoint block's chunks run in sequence in bwd_state_rc, so K > 1 pays only when the blocks
+// fill the chip: D / 64 workgroups per chunk at K = 1, 512 resident at once (two per CU).  Up to one
+// and a half rounds every chunk is a block of its own; up to two, K = 2 fills exactly one round in the
+// same time with half the states kept.  Measured (bwd_state_rc, us, K = 1 / 2 / 3): B1 H2 L256
+// 15 / 28 / 42; B4 H2 L2048 27 / 33 / 45; B4 H3 L2048 (768 workgroups at K = 1) 39 / 47 / 52;
+// B4 H4 L2048 (1024) 51 / 51 / 66; B4 H5 L2048 (1280) 59 / 72 / 69, the whole backward and forward
+// then equal at K = 1 and 3; B4 H6 L2048 69 / 73 / 70, where K = 3 saves 2 % of the whole step in the
+// forward's stores.
+int gdn2_default_state_ckpt(const gdn2_desc* d) {
+  if (!d || d->B < 1 || d->H < 1 || d->L < 1) return 3;
+  const int64_t wgs = (int64_t)d->B * d->H * (d->L / gdn2::T) * (d->D > 64 ? 2 : 1);
+  return wgs <= 768 ? 1 : wgs <= 1024 ? 2 : 3;
+}
+
 // backward workspace: [dv_new | dh_next | dqg | dwp | dkg | dlast | X | Y | EZ (damped) |
 // anchors (bs2 > 64)]
 size_t gdn2_bwd_workspace_bytes(const gdn2_desc* d) {

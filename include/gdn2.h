@@ -213,6 +213,10 @@ int gdn2_wy_stage(const gdn2_desc* d, const float* q, const float* k, const floa
 int gdn2_scores(const gdn2_desc* d, const float* q, const float* k, const float* b, const float* gc,
                 float* aqk, float* akk, void* stream);
 
+/* The checkpoint interval (gdn2_desc.state_ckpt) this library would choose for a training call of
+ * this shape (state_ckpt itself is ignored): 1, 2 or 3.  It changes memory and time, not results. */
+int gdn2_default_state_ckpt(const gdn2_desc* d);
+
 /* ---- the language-model block around the operator ------------------------------------------
  * The element-wise and row-wise passes of the reference's benchmark LM block (GDN2Block; notebook
  * benchmarks/notebooks/all-paths-speed.ipynb, cell 2) between its matrix products, all float32

@@ -118,3 +118,19 @@ def test_checkpoints_are_the_stored_states(L, keep):
     ckpts, o3 = res[3]
     assert torch.equal(ckpts, stored[:, :, keep])
     assert torch.equal(o3, o0)
+
+
+@pytest.mark.parametrize("B,H,L,want", [(1, 2, 256, 1), (3, 4, 2048, 1), (1, 16, 2048, 2), (3, 12, 1024, 3)])
+def test_default_interval_follows_the_grid(B, H, L, want):
+    """state_ckpt=None takes the library's interval for the shape; the gradients are those of every
+    other interval, bit for bit."""
+    from atomic_gdn2 import _lib
+    banner(f"default interval B{B} H{H} L{L}")
+    cfg, D = base_cfg(), 128
+    desc = _lib.training_desc(cfg, B, H, L, D, D ** -0.5, L, None)
+    assert desc.state_ckpt == want
+    arrs = mk_inputs(B, L, H, D, 28, g=0.1, layout="bhld")
+    h0 = (np.random.default_rng(29).normal(size=(B, H, D, D)) * 0.1).astype(np.float32)
+    got, ref = _grad(cfg, D ** -0.5, arrs, h0, None), _grad(cfg, D ** -0.5, arrs, h0, 0)
+    for n in ref:
+        assert torch.equal(got[n], ref[n]), n

@@ -9,7 +9,7 @@ messages.  Tensors are torch tensors on a ROCm device and dtypes are torch dtype
 (``torch.float32`` / ``torch.bfloat16``) where the reference takes jnp ones.
 
 Kernels: ``decode_step`` and the prefill's tail (the tokens after its last full chunk) run the
-token-recurrence kernel (``gdn2_decode``); the prefill's full chunks run the residual-free
+token-recurrence kernels (``gdn2_decode``); the prefill's full chunks run the residual-free
 forward with per-chunk state resets (``gdn2_fwd_reset``: the training forward's kernels, the
 scan zeroing the state entering every chunk whose document differs from the previous chunk's).
 
@@ -206,6 +206,93 @@ def _segment_ids_from_cu_seqlens(cu_seqlens, bsz, L, device):
     return (pos[None, :, None] >= bounds[:, None, :]).sum(dim=-1).to(torch.int32)
 
 
+_ID_TYPES = {torch.int32: 1, torch.int64: 2}          # GDN2_FLAG_INT32, GDN2_FLAG_INT64
+
+
+def _mixed_chunks(seg, n_full, bt):
+    """(B, n_full): whether a full chunk holds more than one document id."""
+    ids = seg[:, :n_full * bt].reshape(seg.shape[0], n_full, bt)
+    return ~(ids == ids[:, :, :1]).all(dim=-1)
+
+
+def _prep_native(g, seg, check_bad, B, H, L, D, bt):
+    """Reset bytes of the chunks and of the tail's tokens (None without ids), and a function that
+    waits for the statistics: (min g, max g, whether a boundary lies inside a full chunk).  One kernel
+    (gdn2_prefill_prep); the statistics travel to pinned memory behind it, so waiting for them does
+    not wait for what is enqueued after."""
+    dev = g.device
+    n_full = L // bt
+    n_stats = 2 * _lib.PREP_G_PARTS + (B * n_full if seg is not None else 0)
+    dev_stats = torch.empty(n_stats, dtype=torch.float32, device=dev)
+    flags = tflags = None
+    if seg is not None:
+        seg = seg.contiguous()
+        if n_full:
+            flags = torch.empty((B, H, n_full * bt // 64), dtype=torch.uint8, device=dev)
+        if L % bt:
+            tflags = torch.empty((B, L % bt), dtype=torch.uint8, device=dev)
+    with torch.cuda.device(dev):
+        _lib.check(_lib.lib().gdn2_prefill_prep(
+            B, H, L, D, bt, int(g.dtype == torch.bfloat16), _lib.ptr(g), 0 if seg is None else _ID_TYPES[seg.dtype],
+            _lib.ptr(seg), _lib.ptr(dev_stats), _lib.ptr(flags), _lib.ptr(tflags), _lib.stream_handle(dev)),
+            "gdn2_prefill_prep")
+        host = torch.empty(n_stats, dtype=torch.float32, pin_memory=True)
+        host.copy_(dev_stats, non_blocking=True)
+        done = torch.cuda.Event()
+        done.record()
+
+    def stats():
+        done.synchronize()
+        part = host[:2 * _lib.PREP_G_PARTS].view(-1, 2)
+        return (float(part[:, 0].min()), float(part[:, 1].max()),
+                check_bad and bool(host[2 * _lib.PREP_G_PARTS:].any()))
+    return flags, tflags, stats
+
+
+def _prep_torch(g, seg, check_bad, B, H, L, D, bt):
+    """_prep_native in torch operations."""
+    n_full, dev = L // bt, g.device
+    L_full = n_full * bt
+    flags = tflags = None
+    if seg is not None and n_full > 0:
+        first = seg[:, :L_full:bt]                                    # (B, n_full) id at each chunk start
+        chg = torch.zeros_like(first, dtype=torch.bool)
+        chg[:, 1:] = first[:, 1:] != first[:, :-1]
+        per64 = torch.zeros((B, L_full // 64), dtype=torch.uint8, device=dev)
+        per64[:, ::bt // 64] = chg.to(torch.uint8)                    # the chunk's first 64-token part
+        flags = per64[:, None, :].expand(B, H, L_full // 64).contiguous()
+    if seg is not None and L > L_full:
+        tail = seg[:, L_full:]
+        prev = seg[:, L_full - 1:L - 1] if L_full > 0 else torch.cat([tail[:, :1], tail[:, :-1]], dim=1)
+        tflags = (tail != prev).to(torch.uint8).contiguous()
+
+    def stats():
+        lo, hi = (float(x) for x in torch.aminmax(g)) if L > 0 else (0.0, 0.0)
+        return lo, hi, check_bad and bool(_mixed_chunks(seg, n_full, bt).any())
+    return flags, tflags, stats
+
+
+def _run_prefill(xs, in_dtype, cfg, scale, h, flags, tflags, sc, B, H, L, D):
+    """The full chunks, then the tail: (o, final state)."""
+    dev = xs[0].device
+    L_full = L // cfg.bt * cfg.bt
+    o = torch.empty((B, H, L, D), dtype=torch.float32, device=dev)
+    L_ = _lib.lib()
+    if L_full > 0:
+        desc = _lib.make_desc(cfg, B, H, L_full, D, scale, seq_ld=L)
+        hf = torch.empty((B, H, D, D), dtype=torch.float32, device=dev)
+        with torch.cuda.device(dev):
+            ws = torch.empty(L_.gdn2_fwd_workspace_bytes(ctypes.byref(desc), 0), dtype=torch.uint8, device=dev)
+            _lib.check(L_.gdn2_fwd_reset(ctypes.byref(desc), in_dtype, *map(_lib.ptr, xs), _lib.ptr(h),
+                                         _lib.ptr(flags), _lib.ptr(o), _lib.ptr(hf), _lib.ptr(ws),
+                                         _lib.stream_handle(dev)), "gdn2_fwd_reset")
+        h = hf
+    if L > L_full:
+        st = None if h is None else h.to(_torch_dtype(sc)).contiguous()
+        h = _run_decode(xs, in_dtype, B, H, D, L - L_full, L, scale, st, sc, o, 0, reset=tflags, offset=L_full * D)
+    return o, h
+
+
 def chunk_forward_inference(q=None, k=None, v=None, w=None, b=None, g=None,
                             scale: float = 1.0, cfg=None,
                             h0=None, segment_ids=None, cu_seqlens=None,
@@ -234,54 +321,47 @@ def chunk_forward_inference(q=None, k=None, v=None, w=None, b=None, g=None,
     sc = _state_code(state_dtype)
     bt = cfg.bt
     n_full = L // bt
-    L_full = n_full * bt
-    r_tail = L - L_full
     scale = float(scale)
     dev = q.device
     g_max_abs = float(cfg.g_max)
     # The domain of g and the document boundaries are checked on the device and read back in one
-    # synchronisation; g is clamped to <= 0 (as on the decode path) only when some g > 0.
-    stats = []
-    if L > 0:
-        g_lo, g_hi = torch.aminmax(g)
-        stats += [g_lo.float(), g_hi.float()]
-    bad = None
-    if segment_ids is not None and n_full > 0:
-        seg_tok = torch.as_tensor(segment_ids, device=dev).reshape(bsz, L)[:, :L_full]
-        per_chunk_first = seg_tok[:, ::bt]
-        same = seg_tok.reshape(bsz, n_full, bt) == per_chunk_first[:, :, None]
-        bad = ~same.all(dim=-1)
-        stats.append(bad.any().float().to(dev))
+    # synchronisation, while the prefill itself is already running: g is clamped to <= 0 (as on the
+    # decode path) only when some g > 0, and the kernels then run again.
     both = segment_ids is not None and cu_seqlens is not None
+    check_bad = segment_ids is not None and n_full > 0
     if cu_seqlens is not None and not both:
         segment_ids = _segment_ids_from_cu_seqlens(cu_seqlens, bsz, L, dev)
-    seg = None if segment_ids is None or both else torch.as_tensor(segment_ids, device=dev).reshape(bsz, L)
-    # the reset bytes are formed before the synchronisation, so that the device is not left idle
-    # while the host builds them after it
-    flags = tflags = None
-    if seg is not None and n_full > 0:
-        sc_ids = seg[:, :L_full:bt]                                   # (B, n_full) id at each chunk start
-        chg = torch.zeros_like(sc_ids, dtype=torch.bool)
-        chg[:, 1:] = sc_ids[:, 1:] != sc_ids[:, :-1]
-        per64 = torch.zeros((bsz, L_full // 64), dtype=torch.uint8, device=dev)
-        per64[:, ::bt // 64] = chg.to(torch.uint8)                    # the chunk's first 64-token half
-        flags = per64[:, None, :].expand(bsz, H, L_full // 64).contiguous()
-    if seg is not None and r_tail > 0:
-        tail = seg[:, L_full:]
-        prev = seg[:, L_full - 1:L - 1] if L_full > 0 else torch.cat([tail[:, :1], tail[:, :-1]], dim=1)
-        tflags = (tail != prev).to(torch.uint8).contiguous()
-    vals = torch.stack([x.to(dev) for x in stats]).tolist() if stats else []
+    seg = None if segment_ids is None else torch.as_tensor(segment_ids, device=dev).reshape(bsz, L)
+    runs = L > 0 and D in (64, 128) and dev.type == "cuda"
+    xs = None
+    if runs:
+        for t, n in zip((k, v, w, b, g), "kvwbg"):
+            if t.device != dev:
+                raise ValueError(f"{n} is on {t.device}, q on {dev}")
+        xs, in_dtype = _inputs_for_kernel((q, k, v, w, b, g))
+        xs[5] = _aligned(xs[5])
+    # (document ids of other integer or float types are formed by torch operations)
+    prep = _prep_native if runs and (seg is None or seg.dtype in _ID_TYPES) else _prep_torch
+    flags, tflags, stats = prep(g if xs is None else xs[5], seg, check_bad, bsz, H, L, D, bt)
+    o = h = None
+    err = None
+    if runs and not both:
+        hin = None if h0 is None else h0.to(torch.float32).to(dev).contiguous()
+        try:
+            o, h = _run_prefill(xs, in_dtype, cfg, scale, hin, flags, tflags, sc, bsz, H, L, D)
+        except (ValueError, _lib.Gdn2Error) as e:
+            err = e                              # g's domain and the boundaries are reported first
+    lo, hi, has_bad = stats()
     # errors in the reference's order: g's domain, a boundary inside a chunk, both id forms
     if L > 0:
         # the layer's domain is [-g_max, 0] (NaN compares false, as in the reference)
-        if min(vals[0], 0.0) < -g_max_abs - 1e-6:
+        if min(lo, 0.0) < -g_max_abs - 1e-6:
             raise ValueError(
                 f"g outside the layer domain: min(g) < -g_max={g_max_abs} "
                 "(the layer constructs g = -min(softplus(...), g_max); clamp or "
                 "fix the projection before calling)")
-        if vals[1] > 0:
-            g = torch.clamp(g, max=0.0)
-    if bad is not None and vals[-1] > 0:
+    if has_bad:
+        bad = _mixed_chunks(seg, n_full, bt)
         b_idx, c_idx = (int(x) for x in torch.nonzero(bad)[0])
         raise ValueError(
             f"document boundary inside chunk {c_idx} of batch row "
@@ -290,29 +370,16 @@ def chunk_forward_inference(q=None, k=None, v=None, w=None, b=None, g=None,
             "chunk_forward_inference (chunk-granularity resets only)")
     if both:
         raise ValueError("pass either segment_ids or cu_seqlens, not both")
-
-    h = None if h0 is None else h0.to(torch.float32)
-    o = None
     if L > 0:
         _check_head_dim(D)
         _check_device(q)
-        xs, in_dtype = _inputs_for_kernel((q, k, v, w, b, g))
-        h = None if h is None else h.to(dev).contiguous()
-        o = torch.empty((bsz, H, L, D), dtype=torch.float32, device=dev)
-        L_ = _lib.lib()
-        if n_full > 0:
-            desc = _lib.make_desc(cfg, bsz, H, L_full, D, scale, seq_ld=L)
-            hf = torch.empty((bsz, H, D, D), dtype=torch.float32, device=dev)
-            with torch.cuda.device(dev):
-                ws = torch.empty(L_.gdn2_fwd_workspace_bytes(ctypes.byref(desc), 0), dtype=torch.uint8, device=dev)
-                _lib.check(L_.gdn2_fwd_reset(ctypes.byref(desc), in_dtype, *map(_lib.ptr, xs), _lib.ptr(h),
-                                             _lib.ptr(flags), _lib.ptr(o), _lib.ptr(hf), _lib.ptr(ws),
-                                             _lib.stream_handle(dev)), "gdn2_fwd_reset")
-            h = hf
-        if r_tail > 0:
-            st = None if h is None else h.to(_torch_dtype(sc)).contiguous()
-            h = _run_decode(xs, in_dtype, bsz, H, D, r_tail, L, scale, st, sc, o, 0, reset=tflags,
-                            offset=L_full * D)
+        if err is not None:
+            raise err
+        if hi > 0:
+            xs[5] = torch.clamp(xs[5], max=0.0)
+            o, h = _run_prefill(xs, in_dtype, cfg, scale, hin, flags, tflags, sc, bsz, H, L, D)
+    else:
+        h = None if h0 is None else h0.to(torch.float32)
     if h is None:
         h = torch.zeros((bsz, H, D, D), dtype=torch.float32, device=dev)
     if stability_tau is not None:

@@ -412,6 +412,29 @@ int gdn2_decode_flags(const gdn2_decode_desc* d, int flag_type, const void* q, c
   return GDN2_OK;
 }
 
+static_assert(GDN2_PREP_G_PARTS == gdn2::PREP_G_BLOCKS, "header constant");
+
+int gdn2_prefill_prep(int B, int H, int L, int D, int bt, int in_dtype, const void* g, int seg_type,
+                      const void* seg, float* stats, uint8_t* flags, uint8_t* tail_flags, void* stream) {
+  if (B < 1 || H < 1 || L < 1 || D < 4 || D % 4 || bt < gdn2::T || bt % gdn2::T)
+    return fail(GDN2_ERR_INVALID, "bad shape");
+  if (in_dtype != 0 && in_dtype != 1) return fail(GDN2_ERR_INVALID, "in_dtype must be 0 (fp32) or 1 (bf16)");
+  if (seg && seg_type != GDN2_FLAG_INT32 && seg_type != GDN2_FLAG_INT64)
+    return fail(GDN2_ERR_INVALID, "document ids are int32 or int64");
+  if (!g || !stats || (reinterpret_cast<uintptr_t>(g) & 15)) return fail(GDN2_ERR_INVALID, "null or misaligned pointer");
+  gdn2::PrefillPrepArgs a{};
+  a.n_full = L / bt;
+  if (seg && ((a.n_full > 0 && !flags) || (L % bt && !tail_flags))) return fail(GDN2_ERR_INVALID, "null flag pointer");
+  if ((int64_t)B * (a.n_full + 1) > (int64_t(1) << 30)) return fail(GDN2_ERR_UNSUPPORTED, "too many chunks");
+  a.g = g; a.seg = seg; a.stats = stats; a.flags = flags; a.tail_flags = tail_flags;
+  a.n_g = (size_t)B * H * L * D;
+  a.g_bf16 = in_dtype; a.seg64 = seg_type == GDN2_FLAG_INT64;
+  a.B = B; a.H = H; a.L = L; a.bt = bt;
+  const hipError_t e = gdn2::launch_prefill_prep(a, reinterpret_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "prefill prep launch");
+  return GDN2_OK;
+}
+
 int gdn2_fwd_reset(const gdn2_desc* d, int in_dtype, const void* q, const void* k, const void* v,
                    const void* w, const void* b, const void* g, const float* h0, const uint8_t* chunk_reset,
                    float* o, float* h_final, void* workspace, void* stream) {

@@ -240,6 +240,20 @@ struct DecodeArgs {
 
 hipError_t launch_decode(int D, const DecodeArgs& a, int n_bh, hipStream_t s);
 
+// Statistics and reset flags of a prefill (gdn2_prefill.hip).  g: n_g elements (a multiple of 4),
+// fp32 or bfloat16 bits; seg: null or B x L document ids (int32 / int64).  stats: PREP_G_BLOCKS pairs
+// (min, max of g over a part), then (with seg) per (batch row, full chunk) 1 when it holds more than
+// one id; flags: (B, H, n_full bt / 64); tail_flags: (B, L - n_full bt).
+constexpr int PREP_G_BLOCKS = 512;
+struct PrefillPrepArgs {
+  const void *g, *seg;
+  float* stats;
+  uint8_t *flags, *tail_flags;
+  size_t n_g;
+  int g_bf16, seg64, B, H, L, bt, n_full;
+};
+hipError_t launch_prefill_prep(const PrefillPrepArgs& a, hipStream_t s);
+
 // Anchors of the diagonal blocks wider than a 64-token part (bs2 = 64 B, B = 2 or 4 parts; kind-2
 // pieces): for part j of a block, in the part's own gc frame (gc restarts at every part),
 //   anc[(part, 0, d)] = gc of the block's first row  = gc_0[0][d] - sum_{i<j} gl_i[d],

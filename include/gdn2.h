@@ -167,6 +167,19 @@ int gdn2_decode(const gdn2_decode_desc* d, const void* q, const void* k, const v
                 const float* dt_bias, const uint8_t* reset, const void* state_in, void* o,
                 void* state_out, void* stream);
 
+/* Statistics and reset flags of a prefill, before gdn2_fwd_reset and gdn2_decode.  g (B,H,L,D) fp32
+ * (in_dtype 0) or bfloat16 bits (1), 16-byte aligned; seg NULL or B*L document ids, int32
+ * (GDN2_FLAG_INT32) or int64 (GDN2_FLAG_INT64).  With n_full = L / bt full chunks:
+ *   stats: GDN2_PREP_G_PARTS pairs (min, max of g over a part; NaN propagates), then, with seg,
+ *     B*n_full floats: 1 when the chunk's ids are not all equal, else 0;
+ *   flags (seg and n_full > 0): B*H*n_full*bt/64 bytes for gdn2_fwd_reset, set on a chunk whose
+ *     first id differs from the previous chunk's;
+ *   tail_flags (seg and L > n_full*bt): B*(L - n_full*bt) bytes for gdn2_decode, set on a token whose
+ *     id differs from the previous token's. */
+#define GDN2_PREP_G_PARTS 512
+int gdn2_prefill_prep(int B, int H, int L, int D, int bt, int in_dtype, const void* g, int seg_type,
+                      const void* seg, float* stats, uint8_t* flags, uint8_t* tail_flags, void* stream);
+
 /* gdn2_decode with the reset flags in the caller's own type: GDN2_FLAG_BYTE as gdn2_decode (set
  * when nonzero); GDN2_FLAG_INT32 set when > 0; GDN2_FLAG_INT64 set when > 0 after a cast to
  * int32.  B*n_tok flags, or NULL. */

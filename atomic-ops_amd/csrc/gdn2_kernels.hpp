@@ -157,6 +157,7 @@ struct ScanFwdArgs {
   int nc, n_bh, ckpt;
   Cfg cfg;
   const uint8_t* reset;
+  int copies;      // set at launch: workgroups per slice, each computing its share of o (gdn2_scan.hip)
 };
 
 // Chunk-parallel output: o = san(s Qg h_pre + Aqk v_new), o row-major (T x D per chunk).

@@ -81,8 +81,8 @@ struct OutOps {
 constexpr int SCAN_SPIN_MAX = 1 << 22;
 // One increment per wave: lane 0 alone issues the add (an add from every active lane would
 // count the wave's active lanes).
-__device__ __forceinline__ void lds_release_add(unsigned* ctr) {
-  if (lane_id() == 0) __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+__device__ __forceinline__ void lds_release_add(unsigned* ctr, unsigned n = 1u) {
+  if (lane_id() == 0) __hip_atomic_fetch_add(ctr, n, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 // Waits until *ctr >= target; ok turns false (and stays false, so later waits return at once)
 // when the spin budget runs out.  SLEEP: pause between polls (the output waves, which wait
@@ -122,7 +122,7 @@ __device__ __forceinline__ void lds_acquire_wait_each(unsigned* ctr, unsigned ta
 struct ScanFwdShared {
   unsigned cbar;           // chain syncs, 4 per sync point: k = 0 after the initial state is in
                            // LDS, k = 2 c + 1 after chunk c's window A, k = 2 c + 2 after its B
-  unsigned odone[4];       // output wave J's releases: 1 per chunk
+  unsigned odone[4];       // output wave J: the chunks before this one are released
 };
 // cbar once sync point k has passed
 __device__ __forceinline__ unsigned cbar_at(int k) { return 4u * (unsigned)(k + 1); }
@@ -131,13 +131,23 @@ __device__ __forceinline__ unsigned cbar_at(int k) { return 4u * (unsigned)(k + 
 // after each part j < G - 1 as the damped state h_d(j+1) = state_update(h_d(j), gamma,
 // (1 - eps) Kg^T v_new) (h_d(0) = h), from which the next part's v_new is computed (the output
 // and the state update keep h).
-template <int D, int MODE, bool OUT>
+// Copies (SPLIT): with few (batch, head)s the launch leaves CUs idle while the output's MFMAs slow the
+// chain on the SIMDs they share.  a.copies workgroups then run each slice's chain, with the same
+// bits, and copy p computes the output of the chunks c = p mod copies only: the chain meets the
+// output's MFMAs in one chunk of copies, and they have that many chunks' time to run in.  Copy 0 alone
+// writes the state, h_pre and v_new.  Measured (scan_fwd, us, 1 / 2 / 4 copies): B1 H6 L1024 43.1 / 40.2 /
+// 38.5, B4 H2 L2048 79.9 / 74.7 / 74.6, the default configuration's B4 H2 L4096 164 / 155 / 152, B1 H6
+// L8192 without a residual 290 / - / 258; more workgroups than CUs cost a second round (B4 H3 L2048
+// 79 / 75 / 138).
+template <int D, int MODE, bool OUT, bool SPLIT>
 __device__ __forceinline__ void scan_fwd_chain(const ScanFwdArgs& a, ScanFwdShared* sh, float4* sH, float4* sHd,
                                                float4* sV, float* sTrK) {
   constexpr int NH = D / 16, NVB = D / 16, NJ = NH / 4;
   const float clip = a.cfg.clip;
   const int nc = a.nc;
-  const int lin = xcd_remap(gridDim.x);
+  const int lin0 = xcd_remap(gridDim.x);
+  const int lin = SPLIT ? lin0 / a.copies : lin0;
+  const bool writes = !SPLIT || lin0 % a.copies == 0;
   // (batch, head)s in reverse order: the WY build writes them in ascending order, so the first
   // workgroups read the lines written last, the likeliest to be still cached (when the grid
   // takes several rounds, config 4: about -1 % of the scan; config 2: -0.9 us)
@@ -210,7 +220,7 @@ __device__ __forceinline__ void scan_fwd_chain(const ScanFwdArgs& a, ScanFwdShar
     float4* sHc = sH + buf * NH * WAVE;            // h_pre of this chunk
     float4* sHn = sH + (1 - buf) * NH * WAVE;      // h_pre of the next one
     float4* sVc = sV + buf * 4 * WAVE;
-    if (a.h_pre_f && c == ck_next) {
+    if (writes && a.h_pre_f && c == ck_next) {
 #pragma unroll
       for (int j = 0; j < NJ; ++j)
         stg4(a.h_pre_f + ((size_t)bh * ckb.nblk + ck_slot) * D * D + frag_blk(vb, kt(j), D) + 4 * l, f4_to_float4(h[j]));
@@ -256,7 +266,7 @@ __device__ __forceinline__ void scan_fwd_chain(const ScanFwdArgs& a, ScanFwdShar
     // the output waves have released chunk c - 2, which used this v_new buffer
     if constexpr (OUT) lds_acquire_wait_each<4>(sh->odone, (unsigned)(c > 1 ? c - 1 : 0), odone_seen, ok);
     sVc[w * WAVE + l] = vn;
-    if (a.v_new_f) stg4(a.v_new_f + tb + frag_blk(vb, w, T) + 4 * l, vn);
+    if (writes && a.v_new_f) stg4(a.v_new_f + tb + frag_blk(vb, w, T) + 4 * l, vn);
     nx.uu = ld4(a.uT_f + tbn + frag_blk(vb, w, T) + 4 * l);
     lds_release_add(&sh->cbar);
     lds_acquire_wait<false>(&sh->cbar, cbar_at(2 * c + 1), ok);
@@ -327,6 +337,7 @@ __device__ __forceinline__ void scan_fwd_chain(const ScanFwdArgs& a, ScanFwdShar
     step(B, c + 1, A, c + 2, std::true_type{});
   }
   if (c < nc) step(A, c, B, c + 1, std::false_type{});
+  if (!writes) return;
 #pragma unroll
   for (int j = 0; j < NJ; ++j)
 #pragma unroll
@@ -336,13 +347,14 @@ __device__ __forceinline__ void scan_fwd_chain(const ScanFwdArgs& a, ScanFwdShar
 // Output wave J (wave 4 + J).  J is a compile-time parameter: the causal Aqk v_new chain's
 // length depends on it, and a runtime branch between the MFMAs of a chain would let the
 // compiler copy the accumulator at the merge point, right after an (opaque) asm MFMA.
-template <int D, int MODE, int J>
+template <int D, int MODE, int J, bool SPLIT>
 __device__ __forceinline__ void scan_fwd_out(const ScanFwdArgs& a, ScanFwdShared* sh, const float4* sH,
                                              const float4* sV) {
   constexpr int NH = D / 16, NVB = D / 16;
   const float clip = a.cfg.clip, scale = a.cfg.scale;
   const int nc = a.nc;
-  const int lin = xcd_remap(gridDim.x);
+  const int lin0 = xcd_remap(gridDim.x), stride = SPLIT ? a.copies : 1;
+  const int lin = SPLIT ? lin0 / stride : lin0, c_first = SPLIT ? lin0 % stride : 0;
   const int vb = lin % NVB, bh = a.n_bh - 1 - lin / NVB, c0 = 16 * vb;   // as the chain waves
   const int l = lane_id(), r = l & 15, g = l >> 4;
   auto base = [&](int c) { return (size_t)bh * nc + (c < nc ? c : nc - 1); };
@@ -356,7 +368,7 @@ __device__ __forceinline__ void scan_fwd_out(const ScanFwdArgs& a, ScanFwdShared
       if (u <= J) op.aq[u] = ld4(a.aqk_f + sb + frag_blk(J, u, T) + 4 * l);
   };
   auto step = [&](const OutOps<NH>& op, int c, OutOps<NH>& nx, int cn, auto odd) {
-    constexpr int buf = decltype(odd)::value ? 1 : 0;
+    const int buf = SPLIT ? c & 1 : (decltype(odd)::value ? 1 : 0);
     const size_t tbn = base(cn) * T * D, sbn = base(cn) * T * T;
     // this chunk's h_pre and v_new are complete once its window-A sync has passed
     lds_acquire_wait<true>(&sh->cbar, cbar_at(2 * c + 1), ok);
@@ -365,7 +377,8 @@ __device__ __forceinline__ void scan_fwd_out(const ScanFwdArgs& a, ScanFwdShared
     for (int kb = 0; kb < NH; ++kb) hb[kb] = sH[buf * NH * WAVE + kb * WAVE + l];
 #pragma unroll
     for (int u = 0; u < 4; ++u) vv[u] = u <= J ? sV[buf * 4 * WAVE + u * WAVE + l] : make_float4(0.f, 0.f, 0.f, 0.f);
-    lds_release_add(&sh->odone[J]);    // the release waits for the reads above
+    // the release waits for the reads above; the chunks before this wave's next one are released too
+    lds_release_add(&sh->odone[J], SPLIT ? (unsigned)stride : 1u);
     f4 acc = {0.f, 0.f, 0.f, 0.f}, acc2 = {0.f, 0.f, 0.f, 0.f};
     if constexpr (MODE == DOT_HIGHEST) {
 #pragma unroll
@@ -410,16 +423,16 @@ __device__ __forceinline__ void scan_fwd_out(const ScanFwdArgs& a, ScanFwdShared
                      sanitize(scale * acc[2] + acc2[2], clip), sanitize(scale * acc[3] + acc2[3], clip)));
   };
   OutOps<NH> A, B;
-  load_all(A, 0);
-  int c = 0;
-  for (; c + 1 < nc; c += 2) {
-    step(A, c, B, c + 1, std::false_type{});
-    step(B, c + 1, A, c + 2, std::true_type{});
+  int c = c_first;
+  load_all(A, c);
+  for (; c + stride < nc; c += 2 * stride) {
+    step(A, c, B, c + stride, std::false_type{});
+    step(B, c + stride, A, c + 2 * stride, std::true_type{});
   }
-  if (c < nc) step(A, c, B, c + 1, std::false_type{});
+  if (c < nc) step(A, c, B, c + stride, std::false_type{});
 }
 
-template <int D, int MODE, bool OUT>
+template <int D, int MODE, bool OUT, bool SPLIT>
 __global__ __launch_bounds__(8 * WAVE) void scan_fwd_kernel(ScanFwdArgs a) {
   constexpr int NH = D / 16;
   __shared__ float4 sH[2 * NH * WAVE];     // h_pre by chunk parity, [buffer][key tile][lane]
@@ -429,19 +442,21 @@ __global__ __launch_bounds__(8 * WAVE) void scan_fwd_kernel(ScanFwdArgs a) {
   __shared__ ScanFwdShared sh;
   if (threadIdx.x == 0) {
     sh.cbar = 0;
-    sh.odone[0] = sh.odone[1] = sh.odone[2] = sh.odone[3] = 0;
+    // the chunks before a copy's first one need no release
+    const unsigned first = SPLIT ? (unsigned)(xcd_remap(gridDim.x) % a.copies) : 0u;
+    sh.odone[0] = sh.odone[1] = sh.odone[2] = sh.odone[3] = first;
   }
   __syncthreads();
   if constexpr (OUT) {
     switch (wave_id()) {
-      case 4: scan_fwd_out<D, MODE, 0>(a, &sh, sH, sV); break;
-      case 5: scan_fwd_out<D, MODE, 1>(a, &sh, sH, sV); break;
-      case 6: scan_fwd_out<D, MODE, 2>(a, &sh, sH, sV); break;
-      case 7: scan_fwd_out<D, MODE, 3>(a, &sh, sH, sV); break;
-      default: scan_fwd_chain<D, MODE, OUT>(a, &sh, sH, sHd, sV, sTrK + wave_id() * 16 * TRP); break;
+      case 4: scan_fwd_out<D, MODE, 0, SPLIT>(a, &sh, sH, sV); break;
+      case 5: scan_fwd_out<D, MODE, 1, SPLIT>(a, &sh, sH, sV); break;
+      case 6: scan_fwd_out<D, MODE, 2, SPLIT>(a, &sh, sH, sV); break;
+      case 7: scan_fwd_out<D, MODE, 3, SPLIT>(a, &sh, sH, sV); break;
+      default: scan_fwd_chain<D, MODE, OUT, SPLIT>(a, &sh, sH, sHd, sV, sTrK + wave_id() * 16 * TRP); break;
     }
   } else {
-    if (wave_id() < 4) scan_fwd_chain<D, MODE, OUT>(a, &sh, sH, sHd, sV, sTrK + wave_id() * 16 * TRP);
+    if (wave_id() < 4) scan_fwd_chain<D, MODE, OUT, SPLIT>(a, &sh, sH, sHd, sV, sTrK + wave_id() * 16 * TRP);
   }
 }
 
@@ -667,16 +682,23 @@ __global__ __launch_bounds__(8 * WAVE) void scan_bwd_kernel(ScanBwdArgs a) {
   else scan_bwd_role<D, MODE, false, true>(a, sDH, sDB, sTr, sWT, sTrs);
 }
 
+template <int D, int MODE>
+static void scan_fwd_launch(ScanFwdArgs a, hipStream_t s) {
+  // copies of each slice while they still get a CU each (one workgroup fills a CU's registers)
+  const int slices = a.n_bh * (D / 16);
+  const int r = 256 / slices;
+  a.copies = !a.o || r < 2 || a.nc < 2 ? 1 : r < 4 ? 2 : 4;
+  const dim3 grid(slices * a.copies), block(512);
+  if (!a.o) hipLaunchKernelGGL((scan_fwd_kernel<D, MODE, false, false>), grid, block, 0, s, a);
+  else if (a.copies == 1) hipLaunchKernelGGL((scan_fwd_kernel<D, MODE, true, false>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((scan_fwd_kernel<D, MODE, true, true>), grid, block, 0, s, a);
+}
+
 hipError_t launch_scan_fwd(int D, const ScanFwdArgs& a, hipStream_t s) {
   dispatch_mode(a.cfg.dot_mode, [&](auto m) {
     constexpr int M = decltype(m)::value;
-    if (a.o) {
-      if (D == 128) hipLaunchKernelGGL((scan_fwd_kernel<128, M, true>), dim3(a.n_bh * 8), dim3(512), 0, s, a);
-      else hipLaunchKernelGGL((scan_fwd_kernel<64, M, true>), dim3(a.n_bh * 4), dim3(512), 0, s, a);
-    } else {
-      if (D == 128) hipLaunchKernelGGL((scan_fwd_kernel<128, M, false>), dim3(a.n_bh * 8), dim3(512), 0, s, a);
-      else hipLaunchKernelGGL((scan_fwd_kernel<64, M, false>), dim3(a.n_bh * 4), dim3(512), 0, s, a);
-    }
+    if (D == 128) scan_fwd_launch<128, M>(a, s);
+    else scan_fwd_launch<64, M>(a, s);
     return 0;
   });
   return hipGetLastError();

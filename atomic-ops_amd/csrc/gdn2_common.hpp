@@ -595,8 +595,18 @@ struct CumsumPass {
     for (int m = 0; m < NV; ++m)
       if (active(m)) {
         const int s = seg(m), cq = col(m);
+        // the run totals above, added in order; read a few at a time (one read per addition would
+        // put its LDS latency on every one of them)
+        constexpr int BATCH = 5;
         float4 off = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int s2 = 0; s2 < s; ++s2) off = add4(off, sTot[s2 * NQP + cq]);
+#pragma unroll
+        for (int b0 = 0; b0 < NSEG - 1; b0 += BATCH) {
+          float4 tot[BATCH];
+#pragma unroll
+          for (int s2 = b0; s2 < b0 + BATCH && s2 < NSEG - 1; ++s2) tot[s2 - b0] = sTot[s2 * NQP + cq];
+#pragma unroll
+          for (int s2 = b0; s2 < b0 + BATCH && s2 < NSEG - 1; ++s2) off = s2 < s ? add4(off, tot[s2 - b0]) : off;
+        }
 #pragma unroll
         for (int i = 0; i < RUN; ++i) st4(sGf + frag_off(s * RUN + i, 4 * cq, 4 * NQP), add4(off, x[m][i]));
       }

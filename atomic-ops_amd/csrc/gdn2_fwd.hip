@@ -273,13 +273,23 @@ __device__ __forceinline__ int tri_row(int t) { return t >= 6 ? 3 : t >= 3 ? 2 :
 //             legs (or, with the lean diagonal, the diagonal blocks exactly);
 //   PM_WIDE   every piece of kind 2 on MFMA (bs2 = 128 / 256, BTL), legs from the anchor buffer.
 enum { PM_TILES = 0, PM_ELEM = 1, PM_WIDE = 2, PM_LEAN = 3 };
-template <int D, int DOT, int PM, typename TIn>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void wy_fwd_kernel(WyFwdArgs a) {
+// NW = 8 (PM_TILES): eight waves per chunk, for launches that leave the chip's wave slots empty, where
+// a chunk's own latency is the launch's time: the waves 4..7 take the second half of each pass's
+// channels in the element-wise steps, the score tiles are spread over all eight, and U is formed
+// beside Wp (from a staging slot of its own).  Every value is formed by the same operations in the
+// same order, so the outputs do not depend on NW.  Measured (us, four -> eight waves): B1 H2 L256 D128
+// 30.8 -> 25.9, B4 H2 L2048 (256 chunks, one per CU) 38.4 -> 33.2, with bf16x3 products 39.7 -> 32.4;
+// past one chunk per CU four waves and three workgroups per CU are the better form (B4 H3 L2048: 41
+// against 57 us, or 44 with two workgroups of eight waves at 128 registers, which spill).
+template <int D, int DOT, int PM, typename TIn, int NW = 4>
+__global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(NW == 8 ? 2 : 3))) void wy_fwd_kernel(WyFwdArgs a) {
   constexpr bool ELEM = PM == PM_ELEM || PM == PM_LEAN, WIDE = PM == PM_WIDE;
   using Lay = WyLayout<D>;
-  constexpr int NT = 256, DC = Lay::DC, NPASS = Lay::NPASS, NKBP = Lay::NKBP, LT = Lay::LT, NKB = D / 16;
-  constexpr int NSLOT = (WY_NTL + 3) / 4;
-  __shared__ __attribute__((aligned(16))) float smem[Lay::TOTAL];
+  constexpr int NT = NW * WAVE, DC = Lay::DC, NPASS = Lay::NPASS, NKBP = Lay::NKBP, LT = Lay::LT, NKB = D / 16;
+  constexpr int NSLOT = (WY_NTL + NW - 1) / NW;
+  constexpr int HF = NW / 4, NKW = NKBP / HF;      // waves per token tile; its k blocks of a pass per wave
+  static_assert(HF == 1 || HF == 2 && NKBP == 2, "one or two waves per token tile");
+  __shared__ __attribute__((aligned(16))) float smem[Lay::TOTAL + (HF == 2 ? 64 * T : 0)];
   float* sG = smem + Lay::OFF_G;
   float* sQ = smem + Lay::OFF_Q;
   float* sKs = smem + Lay::OFF_K;
@@ -301,29 +311,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void w
   const TIn* __restrict__ v = static_cast<const TIn*>(a.v) + tio;
   const TIn* __restrict__ gg = static_cast<const TIn*>(a.g) + tio;
   const int tid = threadIdx.x, wv = wave_id(), l = lane_id(), r = l & 15, g = l >> 4;
-  float* tr = smem + Lay::OFF_TR + wv * 16 * TRP;
-  // elementwise steps: wave wv owns token tile wv, lane (r, g) row 16 wv + r, columns 16 kb + 4 g
-  const int row = 16 * wv + r;
+  // elementwise steps: wave wv owns token tile tt, lane (r, g) row 16 tt + r, columns 16 kb + 4 g of the
+  // k blocks kb = HF j + hf, j < NKW, of each pass
+  const int tt = wv & 3, hf = HF == 2 ? wv >> 2 : 0;
+  const int row = 16 * tt + r;
+  float* tr = HF == 2 ? smem + Lay::TOTAL + wv * 16 * TRP : smem + Lay::OFF_TR + wv * 16 * TRP;
+  static_assert(HF == 1 || 8 * 16 * TRP <= 64 * T, "eight transpose tiles fit in the second staging slot");
 
-  // the pieces of this wave's score tiles t = wv + 4 s (scalar reads, before any memory traffic)
+  // the pieces of this wave's score tiles t = wv + NW s (scalar reads, before any memory traffic)
   Piece pcs[NSLOT];
 #pragma unroll
   for (int s = 0; s < NSLOT; ++s) {
-    const int t = wv + 4 * s < WY_NTL ? wv + 4 * s : 0, ti = tri_row(t), tj = t - ti * (ti + 1) / 2;
+    const int t = wv + NW * s < WY_NTL ? wv + NW * s : 0, ti = tri_row(t), tj = t - ti * (ti + 1) / 2;
     pcs[s] = piece_at(cf.pieces, cf.tile_piece[4 * ti + tj]);
   }
 
   // this pass's inputs: the cumsum's g runs, and q, k, b as the wave's row fragments
   CumsumPass<D, 512, NT, DC / 4> cs;
-  float4 xq[NKBP], xk[NKBP], xb[NKBP];
+  float4 xq[NKW], xk[NKW], xb[NKW];
   auto load_pass = [&](int p) __attribute__((always_inline)) {
     cs.load(gg, DC * p);
 #pragma unroll
-    for (int kb = 0; kb < NKBP; ++kb) {
-      const int o = row * D + DC * p + 16 * kb + 4 * g;
-      xq[kb] = in_ld4(q + o);
-      xk[kb] = in_ld4(k + o);
-      xb[kb] = in_ld4(b + o);
+    for (int j = 0; j < NKW; ++j) {
+      const int o = row * D + DC * p + 16 * (HF * j + hf) + 4 * g;
+      xq[j] = in_ld4(q + o);
+      xk[j] = in_ld4(k + o);
+      xb[j] = in_ld4(b + o);
     }
   };
   load_pass(0);
@@ -331,7 +344,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void w
   f4 accq[NSLOT], acck[NSLOT];
 #pragma unroll
   for (int s = 0; s < NSLOT; ++s) accq[s] = acck[s] = f4{0.f, 0.f, 0.f, 0.f};
-  float4 xT[NKB];     // X^T = (b k e^gc)^T, fragment blocks (kb, wv), staged for Wp after the scores
+  float4 xT[NKB / HF];     // X^T = (b k e^gc)^T, fragment blocks (kb, tt), staged for Wp after the scores
   // ELEM: this thread's elementwise score elements (element m = tid + NT m of the elementwise
   // pieces taken in order), their running sums over d.  At most 12 per thread: the diagonal
   // pieces of bs2 = 64 (3 x 32 x 32) or every piece of bs2 = 8 (36 x 8 x 8).
@@ -339,6 +352,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void w
   auto elementwise = [&](const Piece& pc) {
     return PM == PM_LEAN ? pc.kind != 0 : (lean && pc.kind != 0) || pc.P < 16;
   };
+  static_assert(!ELEM || NW == 4, "12 elements per thread at four waves");
   constexpr int NLEAN = ELEM ? 12 : 1;
   float lq[NLEAN], lk[NLEAN];
 #pragma unroll
@@ -369,29 +383,29 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void w
     // 2. gated fragments (cd_slim.py:17-21): Kg = san(k e^{min(gl - gc, 0)}) as FRAG(Kg) (the
     //    forward scan turns its blocks around itself); Qg = san(q e^{min(gc, 0)}); X = b k e^{min(gc, 0)}
     //    (transposed, kept for Wp).  Staged for the scores: gc (already), q, k, b k.
-    float4 kgv[NKBP], qgv[NKBP], bkv[NKBP];
+    float4 kgv[NKW], qgv[NKW], bkv[NKW];
 #pragma unroll
-    for (int kb = 0; kb < NKBP; ++kb) {
-      const int o = frag_blk(wv, kb, DC) + 4 * l;
+    for (int j = 0; j < NKW; ++j) {
+      const int kb = HF * j + hf, o = frag_blk(tt, kb, DC) + 4 * l;
       const float4 gc = ld4(sG + o), gl = ld4(sG + frag_off(T - 1, 16 * kb + 4 * g, DC));
-      kgv[kb] = san4(mul4(xk[kb], expnp4(sub4(gl, gc))), clip);
+      kgv[j] = san4(mul4(xk[j], expnp4(sub4(gl, gc))), clip);
       const float4 eg = expnp4(gc);
-      qgv[kb] = san4(mul4(xq[kb], eg), clip);
-      bkv[kb] = mul4(xb[kb], xk[kb]);
-      st4(sQ + o, xq[kb]);
-      st4(sKs + o, xk[kb]);
-      st4(sBK + o, bkv[kb]);
-      xT[NKBP * p + kb] = wave_transpose16(tr, mul4(bkv[kb], eg), r, g);
+      qgv[j] = san4(mul4(xq[j], eg), clip);
+      bkv[j] = mul4(xb[j], xk[j]);
+      st4(sQ + o, xq[j]);
+      st4(sKs + o, xk[j]);
+      st4(sBK + o, bkv[j]);
+      xT[NKW * p + j] = wave_transpose16(tr, mul4(bkv[j], eg), r, g);
     }
     // the next pass's loads go out before this pass's stores (the memory counter is in order)
     if (p + 1 < NPASS) load_pass(p + 1);
 #pragma unroll
-    for (int kb = 0; kb < NKBP; ++kb) {
-      const int kg = NKBP * p + kb, d = DC * p + 16 * kb + 4 * g;
-      if (a.kg_f) stg4_keep(a.kg_f + tb + frag_blk(wv, kg, D) + 4 * l, kgv[kb]);
-      if (a.kg) stg4_keep(a.kg + tb + row * D + d, kgv[kb]);
-      if (a.qg_f) stg4_keep(a.qg_f + tb + frag_blk(wv, kg, D) + 4 * l, qgv[kb]);
-      if (a.qg) stg4_keep(a.qg + tb + row * D + d, qgv[kb]);
+    for (int j = 0; j < NKW; ++j) {
+      const int kb = HF * j + hf, kg = NKBP * p + kb, d = DC * p + 16 * kb + 4 * g;
+      if (a.kg_f) stg4_keep(a.kg_f + tb + frag_blk(tt, kg, D) + 4 * l, kgv[j]);
+      if (a.kg) stg4_keep(a.kg + tb + row * D + d, kgv[j]);
+      if (a.qg_f) stg4_keep(a.qg_f + tb + frag_blk(tt, kg, D) + 4 * l, qgv[j]);
+      if (a.qg) stg4_keep(a.qg + tb + row * D + d, qgv[j]);
     }
     if (a.gl && tid < DC) a.gl[(size_t)chunk * D + DC * p + tid] = sG[frag_off(T - 1, tid, DC)];
     // kind-2 anchors of this pass's channels (first row | last row of the diagonal block)
@@ -401,10 +415,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void w
     }
     __syncthreads();
 
-    // 3. scores over this pass's k blocks (scores.py:39-84): tiles t = wv + 4 s
+    // 3. scores over this pass's k blocks (scores.py:39-84): tiles t = wv + NW s
 #pragma unroll
     for (int s = 0; s < NSLOT; ++s) {
-      const int t = wv + 4 * s;
+      const int t = wv + NW * s;
       if (t >= WY_NTL) continue;
       const int ti = tri_row(t), tj = t - ti * (ti + 1) / 2;
       const Piece& pc = pcs[s];
@@ -450,7 +464,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void w
   const float ome = cf.ome, scale = cf.scale;
 #pragma unroll
   for (int s = 0; s < NSLOT; ++s) {
-    const int t = wv + 4 * s;
+    const int t = wv + NW * s;
     if (t >= WY_NTL) continue;
     const int ti = tri_row(t), tj = t - ti * (ti + 1) / 2;
     const int i = 16 * ti + r, j0 = 16 * tj + 4 * g;
@@ -479,7 +493,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void w
     if (a.akk) stg4_keep(a.akk + sb + i * T + j0, ak4);
   }
   // upper tiles (tj > ti): zeros
-  for (int t = wv; t < 16; t += 4) {
+  for (int t = wv; t < 16; t += NW) {
     const int ti = t / 4, tj = t % 4;
     if (tj <= ti) continue;
     const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -530,34 +544,81 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void w
       }
     }
   };
+  // strip tj of a matrix (mat 0: Wp, 1: U; compile-time: no branch in a chain) from its four staged
+  // blocks (tj, kb) of X^T or Y^T
+  auto strip = [&](auto matc, int tj, const float4 (&xbv)[4]) __attribute__((always_inline)) {
+    constexpr int mat = decltype(matc)::value;
+    f4 acc[4];
+#pragma unroll
+    for (int ti = 0; ti < 4; ++ti) acc[ti] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+      for (int ti = kb; ti < 4; ++ti) {
+        const float4 av = ld4(sI + (16 * ti + r) * LT + 16 * kb + 4 * g);
+        if constexpr (mat == 0) mma16_tr<DOT>(acc[ti], xbv[kb], av);
+        else mma16<DOT>(acc[ti], av, xbv[kb]);
+      }
+    drain(acc[0], acc[1], acc[2], acc[3]);
+#pragma unroll
+    for (int ti = 0; ti < 4; ++ti) store_tile(matc, ti, tj, acc[ti]);
+  };
+  using MatW = std::integral_constant<int, 0>;
+  using MatU = std::integral_constant<int, 1>;
+  if constexpr (HF == 2) {
+    // waves 0..3 the strips of Wp, waves 4..7 those of U, four channel tiles at a time; wave
+    // (tt, hf) stages its channel tiles c = hf, 2 + hf of the group
+    float* sY = smem + Lay::TOTAL;
+    float4 xw[2], xv[2];
+    auto load_wv = [&](int m) __attribute__((always_inline)) {
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int o = row * D + 64 * m + 16 * (2 * c + hf) + 4 * g;
+        xw[c] = in_ld4(w + o);
+        xv[c] = in_ld4(v + o);
+      }
+    };
+    if (want_u) load_wv(0);
+    float4 yT[2] = {make_float4(0.f, 0.f, 0.f, 0.f), make_float4(0.f, 0.f, 0.f, 0.f)};
+#pragma unroll
+    for (int m = 0; m < NKB / 4; ++m) {
+      // the transpose tiles lie in the Y slot: every wave turns its blocks around, then they are staged
+      if (want_u) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) yT[c] = wave_transpose16(tr, mul4(xw[c], xv[c]), r, g);
+        if (m + 1 < NKB / 4) load_wv(m + 1);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        st4(sX + frag_blk(2 * c + hf, tt, T) + 4 * l, xT[2 * m + c]);
+        st4(sY + frag_blk(2 * c + hf, tt, T) + 4 * l, yT[c]);
+      }
+      __syncthreads();
+      const float* src = hf ? sY : sX;
+      float4 xbv[4];
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) xbv[kb] = ld4(src + frag_blk(tt, kb, T) + 4 * l);
+      __syncthreads();
+      if (hf == 0) {
+        if (want_w) strip(MatW{}, 4 * m + tt, xbv);
+      } else {
+        if (want_u) strip(MatU{}, 4 * m + tt, xbv);
+      }
+    }
+    return;
+  }
   // strips of four channel tiles at a time (group m): the group's B operands (blocks (tj, kb) of
   // X^T or Y^T) staged in the Akk slot, wave wv computes strip tj = 4 m + wv
   auto products = [&](auto matc, int m, const float4* opT) __attribute__((always_inline)) {
-    constexpr int mat = decltype(matc)::value;     // 0: Wp, 1: U (compile-time: no branch in a chain)
-    {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) st4(sX + frag_blk(c, wv, T) + 4 * l, opT[c]);
-      __syncthreads();
-      const int tj = 4 * m + wv;
-      float4 xbv[4];
+    for (int c = 0; c < 4; ++c) st4(sX + frag_blk(c, wv, T) + 4 * l, opT[c]);
+    __syncthreads();
+    float4 xbv[4];
 #pragma unroll
-      for (int kb = 0; kb < 4; ++kb) xbv[kb] = ld4(sX + frag_blk(wv, kb, T) + 4 * l);
-      __syncthreads();
-      f4 acc[4];
-#pragma unroll
-      for (int ti = 0; ti < 4; ++ti) acc[ti] = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-        for (int ti = kb; ti < 4; ++ti) {
-          const float4 av = ld4(sI + (16 * ti + r) * LT + 16 * kb + 4 * g);
-          if constexpr (mat == 0) mma16_tr<DOT>(acc[ti], xbv[kb], av);
-          else mma16<DOT>(acc[ti], av, xbv[kb]);
-        }
-      drain(acc[0], acc[1], acc[2], acc[3]);
-#pragma unroll
-      for (int ti = 0; ti < 4; ++ti) store_tile(matc, ti, tj, acc[ti]);
-    }
+    for (int kb = 0; kb < 4; ++kb) xbv[kb] = ld4(sX + frag_blk(wv, kb, T) + 4 * l);
+    __syncthreads();
+    strip(matc, 4 * m + wv, xbv);
   };
   // w and v of one strip group (the wave's row fragments), for Y = w v: group 0's loads go out
   // before the Wp products, each next group's before the current group's U products
@@ -573,7 +634,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void w
   if (want_u) load_wv(0);
   if (want_w) {
 #pragma unroll
-    for (int m = 0; m < NKB / 4; ++m) products(std::integral_constant<int, 0>{}, m, xT + 4 * m);
+    for (int m = 0; m < NKB / 4; ++m) products(MatW{}, m, xT + 4 * m);
   }
   if (want_u) {
 #pragma unroll
@@ -582,7 +643,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void w
 #pragma unroll
       for (int c = 0; c < 4; ++c) yT[c] = wave_transpose16(tr, mul4(xw[c], xv[c]), r, g);
       if (m + 1 < NKB / 4) load_wv(m + 1);
-      products(std::integral_constant<int, 1>{}, m, yT);
+      products(MatU{}, m, yT);
     }
   }
 }
@@ -790,6 +851,8 @@ hipError_t launch_anchors(int D, const AnchorArgs& a, hipStream_t s, bool bf16_i
   return hipGetLastError();
 }
 
+constexpr int WY_NW8_CHUNKS = 256;      // one chunk per CU (wy_fwd_kernel, NW)
+
 hipError_t launch_wy_fwd(int D, const WyFwdArgs& a, hipStream_t s, bool bf16_inputs) {
   // every piece has side min(bs2, 32) and, past bs2 = 64, kind 2
   const Piece& p0 = a.cfg.pieces.p[0];
@@ -797,13 +860,14 @@ hipError_t launch_wy_fwd(int D, const WyFwdArgs& a, hipStream_t s, bool bf16_inp
   if (pm == PM_WIDE && !a.anc) return hipErrorInvalidValue;
   dispatch_mode(a.cfg.dot_mode, [&](auto m) {
     constexpr int M = decltype(m)::value;
-    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(a.n_chunks), dim3(256), 0, s, a); };
+    auto go = [&](auto kern, int threads = 256) { hipLaunchKernelGGL(kern, dim3(a.n_chunks), dim3(threads), 0, s, a); };
     auto by_pm = [&](auto d, auto tin) {
       constexpr int DD = decltype(d)::value;
       using TI = decltype(tin);
       if (pm == PM_ELEM) go(wy_fwd_kernel<DD, M, PM_ELEM, TI>);
       else if (pm == PM_LEAN) go(wy_fwd_kernel<DD, M, PM_LEAN, TI>);
       else if (pm == PM_WIDE) go(wy_fwd_kernel<DD, M, PM_WIDE, TI>);
+      else if (a.n_chunks <= WY_NW8_CHUNKS) go(wy_fwd_kernel<DD, M, PM_TILES, TI, 8>, 512);
       else go(wy_fwd_kernel<DD, M, PM_TILES, TI>);
     };
     if (bf16_inputs) {

@@ -351,11 +351,25 @@ def usable(block, x, dense, conv, norm):
         return False
     if any((mods[n].bias is None) == (n in _BIASED) for n in _DENSE):
         return False
-    return all(type(p) is torch.nn.Parameter and _ready(p, x.device) for p in block.parameters())
+    d, p, H, M = c.d_model, c.proj_dim, c.n_heads, c.mlp_mult * c.d_model
+    shapes = [(d, p)] * 6 + [(d, H)] + [(p, 4), (p,)] * 3 + [(p,)] * 2 + [(H,)] * 2 + [(p,), (p, d), (d,), (d, M), (d, M), (M, d)]
+    return x.shape[-1] == d and all(
+        type(t) in (torch.Tensor, torch.nn.Parameter) and t.shape == sh and _ready(t, x.device)
+        for t, sh in zip(_tensors(block), shapes))
+
+
+def _tensors(m):
+    """The block's weights in the order the three nodes take them (17, then 2, then 4)."""
+    return (m.q_proj.weight, m.k_proj.weight, m.v_proj.weight, m.erase_gate.weight, m.write_gate.weight, m.out_gate.weight,
+            m.decay_proj.weight, m.q_conv.weight, m.q_conv.bias, m.k_conv.weight, m.k_conv.bias, m.v_conv.weight,
+            m.v_conv.bias, m.erase_gate.bias, m.write_gate.bias, m.decay_proj.bias, m.decay_a,
+            m.mixer_out_norm.scale, m.out_proj.weight,
+            m.mlp_norm.scale, m.gate_proj.weight, m.up_proj.weight, m.down_proj.weight)
 
 
 def norm_usable(module, x, norm):
-    return (_plain(module, norm) and module.eps == _EPS and _usable_input(x) and type(module.scale) is torch.nn.Parameter
+    return (_plain(module, norm) and module.eps == _EPS and _usable_input(x)
+            and type(module.scale) in (torch.Tensor, torch.nn.Parameter) and module.scale.shape == x.shape[-1:]
             and _ready(module.scale, x.device))
 
 
@@ -364,11 +378,8 @@ def rms_norm(module, x):
 
 
 def block_forward(m, x):
-    c = m.cfg
-    *ops, og = _PreMix.apply(
-        c.n_heads, c.d_head, c.g_max, x, m.q_proj.weight, m.k_proj.weight, m.v_proj.weight, m.erase_gate.weight,
-        m.write_gate.weight, m.out_gate.weight, m.decay_proj.weight, m.q_conv.weight, m.q_conv.bias, m.k_conv.weight,
-        m.k_conv.bias, m.v_conv.weight, m.v_conv.bias, m.erase_gate.bias, m.write_gate.bias, m.decay_proj.bias, m.decay_a)
+    c, ws = m.cfg, _tensors(m)
+    *ops, og = _PreMix.apply(c.n_heads, c.d_head, c.g_max, x, *ws[:17])
     o, _ = m.kernel_fn.head_major(*ops)
-    x = _PostMix.apply(o, og, x, m.mixer_out_norm.scale, m.out_proj.weight)
-    return _Mlp.apply(x, m.mlp_norm.scale, m.gate_proj.weight, m.up_proj.weight, m.down_proj.weight)
+    x = _PostMix.apply(o, og, x, *ws[17:19])
+    return _Mlp.apply(x, *ws[19:])

@@ -161,5 +161,9 @@ def test_module_forward_stays_in_charge():
         b = _block(cfg, op)
         b.mlp_norm.scale = torch.nn.Parameter(flat[1:])
         assert not lm_kernels.usable(b, x, *kinds)
+        b = _block(cfg, op)
+        del b.mlp_norm.scale                   # a plain tensor in a parameter's place, of another shape
+        b.mlp_norm.scale = torch.zeros(32)
+        assert not lm_kernels.usable(b, x, *kinds)
     finally:
         lm_kernels._usable_input = real

@@ -124,8 +124,12 @@ def _weight_grad(x, dy):
 
 
 def _vjp_through(ref, inputs, needs, grads):
-    """Gradients of ref(*inputs) for a backward that is itself differentiated."""
+    """Gradients of ref(*inputs) for a backward that is itself differentiated.  They are taken at
+    aliases of the inputs: an input may be computed from another one (the operator's o and the
+    gate's logits from x) or appear twice (a tied weight), and each gradient is this node's own
+    share, without the paths that lie outside it."""
     with torch.enable_grad():
+        inputs = [x.view_as(x) for x in inputs]
         outs = ref(*inputs)
         outs = outs if isinstance(outs, tuple) else (outs,)
         pairs = [(o, g) for o, g in zip(outs, grads) if g is not None and o.requires_grad]

@@ -78,7 +78,7 @@ def blhd_kernel(cfg, d_head):
         o, _ = fn(*(sw(x) for x in (q, k, v, w, b, g)))
         return o.transpose(1, 2)
 
-    run.head_major = fn       # the operator itself, for callers whose tensors are head-major already
+    lm_kernels.register_operator(run, fn)       # for blocks whose tensors are head-major already
     return run
 
 
@@ -178,7 +178,7 @@ class LM(nn.Module):
         x = self.embed[ids]
         for blk in self.blocks:
             x = blk(x)
-        if (len(self.blocks) and getattr(self.blocks[-1].kernel_fn, "head_major", None) is not None
+        if (len(self.blocks) and lm_kernels.operator_of(self.blocks[-1].kernel_fn) is not None
                 and lm_kernels.norm_usable(self.final_norm, x, RMSNorm)):
             return lm_kernels.rms_norm(self.final_norm, x) @ self.embed.t()
         return self.final_norm(x) @ self.embed.t()

@@ -19,6 +19,8 @@ other dtypes, autocast, hooked or replaced submodules, another mixer) the module
 from __future__ import annotations
 
 import ctypes
+import types
+import weakref
 
 import torch
 import torch.nn.functional as F
@@ -340,12 +342,26 @@ def _usable_input(x):
             and not torch.nn.modules.module._has_any_global_hook())
 
 
+_OPERATORS = weakref.WeakKeyDictionary()    # a (B, L, H, D) mixer -> the operator it stands for
+
+
+def register_operator(mixer, operator):
+    """Declare that the function ``mixer`` of (B, L, H, D) tensors is the HIP operator ``operator`` of
+    head-major ones, so that a block may call the latter.  Kept by the function's identity: a wrapper
+    around the mixer is another mixer, whatever attributes it copied."""
+    _OPERATORS[mixer] = operator
+
+
+def operator_of(mixer):
+    """The head-major operator that mixer was registered for, or None."""
+    return _OPERATORS.get(mixer) if type(mixer) is types.FunctionType else None
+
+
 def usable(block, x, dense, conv, norm):
     """Whether block_forward stands for block.forward(x); dense, conv, norm: the module types that
     the block is built of."""
-    fn = getattr(block.kernel_fn, "head_major", None)
     c = block.cfg
-    if fn is None or not (x.dim() == 3 and _usable_input(x)):
+    if operator_of(block.kernel_fn) is None or not (x.dim() == 3 and _usable_input(x)):
         return False
     if c.d_head not in (64, 128) or c.d_conv != 4 or c.proj_dim > _MAX_C or (c.mlp_mult * c.d_model) % 4:
         return False
@@ -384,6 +400,6 @@ def rms_norm(module, x):
 def block_forward(m, x):
     c, ws = m.cfg, _tensors(m)
     *ops, og = _PreMix.apply(c.n_heads, c.d_head, c.g_max, x, *ws[:17])
-    o, _ = m.kernel_fn.head_major(*ops)
+    o, _ = operator_of(m.kernel_fn)(*ops)
     x = _PostMix.apply(o, og, x, *ws[17:19])
     return _Mlp.apply(x, *ws[19:])

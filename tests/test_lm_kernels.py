@@ -1,6 +1,7 @@
 """The language-model block's HIP passes (lm_kernels) against the same block in torch operations, and
 where the module forward has to stay in charge."""
 import dataclasses
+import functools
 
 import pytest
 import torch
@@ -117,7 +118,7 @@ def test_block_is_the_module_forward():
     leaves = [x] + list(blk.parameters())
     w = torch.randn(2, 192, 128, device="cuda")
     got = [blk(x)] + list(torch.autograd.grad(blk(x), leaves, w))
-    blk.kernel_fn = lambda *a: op(*a)          # no head_major: the module forward
+    blk.kernel_fn = lambda *a: op(*a)          # another mixer: the module forward
     assert not lm_kernels.usable(blk, x, *kinds)
     want = [blk(x)] + list(torch.autograd.grad(blk(x), leaves, w))
     for a, b in zip(got, want):
@@ -165,5 +166,28 @@ def test_module_forward_stays_in_charge():
         del b.mlp_norm.scale                   # a plain tensor in a parameter's place, of another shape
         b.mlp_norm.scale = torch.zeros(32)
         assert not lm_kernels.usable(b, x, *kinds)
+    finally:
+        lm_kernels._usable_input = real
+
+
+def test_a_wrapped_mixer_keeps_the_module_forward():
+    """A mixer built around the operator is another mixer, also where functools.wraps has copied the
+    operator's attributes: its body runs."""
+    from atomic_gdn2 import e2e_lm, lm_kernels
+    cfg = e2e_lm.LMConfig(d_model=64, n_heads=1, d_head=64)
+    op = e2e_lm.blhd_kernel(e2e_lm.operator_cfg(), 64)
+
+    @functools.wraps(op)
+    def half(*a):
+        return 0.5 * op(*a)
+
+    kinds = (e2e_lm.Dense, e2e_lm.CausalDepthwiseConv, e2e_lm.RMSNorm)
+    real = lm_kernels._usable_input
+    lm_kernels._usable_input = lambda x: True           # the device test planted away
+    try:
+        x = torch.zeros(1, 64, 64)
+        assert lm_kernels.usable(_block(cfg, op), x, *kinds)
+        assert not lm_kernels.usable(_block(cfg, half), x, *kinds)
+        assert not lm_kernels.usable(_block(cfg, functools.partial(op)), x, *kinds)
     finally:
         lm_kernels._usable_input = real

@@ -127,6 +127,9 @@ class CausalDepthwiseConv(nn.Module):
         return lm_kernels.conv_ref(x, self.weight, self.bias)
 
 
+lm_kernels.register_modules(Dense, CausalDepthwiseConv, RMSNorm)
+
+
 class GDN2Block(nn.Module):
     def __init__(self, cfg: LMConfig, kernel_fn):
         super().__init__()

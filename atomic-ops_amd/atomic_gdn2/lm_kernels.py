@@ -14,7 +14,7 @@ itself to be differentiated (``create_graph``) recomputes the step from ``_premi
 
 ``usable`` says where this path stands in for the module's own forward: float32 on the GPU, the
 block's own submodule types without hooks, the HIP operator as the mixer.  Everywhere else (the CPU,
-other dtypes, autocast, hooked or replaced submodules, another mixer) the module forward runs.
+other dtypes, autocast, hooked, patched or replaced submodules, another mixer) the module forward runs.
 """
 from __future__ import annotations
 
@@ -332,8 +332,17 @@ def _ready(t, dev):
             and t.numel() > 0)
 
 
+_FORWARDS = {}          # module class -> its own forward
+
+
+def register_modules(*classes):
+    """Declare the module classes a block is built of, with the forwards that block_forward computes."""
+    _FORWARDS.update((c, c.forward) for c in classes)
+
+
 def _plain(m, cls):
-    return type(m) is cls and not any(getattr(m, h) for h in _HOOKS)
+    return (type(m) is cls and cls.forward is _FORWARDS.get(cls) and "forward" not in m.__dict__
+            and not any(getattr(m, h) for h in _HOOKS))
 
 
 def _usable_input(x):
@@ -366,8 +375,8 @@ def usable(block, x, dense, conv, norm):
     if c.d_head not in (64, 128) or c.d_conv != 4 or c.proj_dim > _MAX_C or (c.mlp_mult * c.d_model) % 4:
         return False
     mods = block._modules
-    if not (all(_plain(mods[n], dense) for n in _DENSE) and all(_plain(mods[n], conv) for n in _CONV)
-            and all(_plain(mods[n], norm) and mods[n].eps == _EPS for n in _NORM)):
+    if not (all(_plain(mods.get(n), dense) for n in _DENSE) and all(_plain(mods.get(n), conv) for n in _CONV)
+            and all(_plain(mods.get(n), norm) and mods[n].eps == _EPS for n in _NORM)):
         return False
     if any((mods[n].bias is None) == (n in _BIASED) for n in _DENSE):
         return False

@@ -191,3 +191,31 @@ def test_a_wrapped_mixer_keeps_the_module_forward():
         assert not lm_kernels.usable(_block(cfg, functools.partial(op)), x, *kinds)
     finally:
         lm_kernels._usable_input = real
+
+
+def test_a_patched_submodule_keeps_the_module_forward(monkeypatch):
+    """A submodule whose forward was replaced on the instance or on its class, or that was taken out
+    and replaced by a plain callable, runs as the program has it."""
+    from atomic_gdn2 import e2e_lm, lm_kernels
+    cfg = e2e_lm.LMConfig(d_model=64, n_heads=1, d_head=64)
+    op = e2e_lm.blhd_kernel(e2e_lm.operator_cfg(), 64)
+    kinds = (e2e_lm.Dense, e2e_lm.CausalDepthwiseConv, e2e_lm.RMSNorm)
+    monkeypatch.setattr(lm_kernels, "_usable_input", lambda x: True)        # the device test planted away
+    x = torch.zeros(1, 64, 64)
+    for name in ("q_proj", "v_conv", "mlp_norm"):
+        b = _block(cfg, op)
+        assert lm_kernels.usable(b, x, *kinds)
+        m = getattr(b, name)
+        plain = m.forward
+        m.forward = lambda y: 2.0 * plain(y)
+        assert not lm_kernels.usable(b, x, *kinds)
+        b = _block(cfg, op)
+        delattr(b, name)
+        setattr(b, name, lambda y: y)
+        assert not lm_kernels.usable(b, x, *kinds)
+        with monkeypatch.context() as mp:
+            cls = type(m)
+            f = cls.forward
+            mp.setattr(cls, "forward", lambda self, y: 2.0 * f(self, y))
+            assert not lm_kernels.usable(_block(cfg, op), x, *kinds)
+            assert name != "mlp_norm" or not lm_kernels.norm_usable(_block(cfg, op).mlp_norm, x, e2e_lm.RMSNorm)

@@ -748,6 +748,11 @@ int gdn2_lm_columns(int split, float* const parts[], const int32_t widths[], int
   return lm_done(gdn2::launch_lm_columns(a, split != 0, reinterpret_cast<hipStream_t>(stream)), "lm columns launch");
 }
 
+int gdn2_debug_scan_copies(int n_bh, int D, int nc, int in_place) {
+  if (n_bh < 1 || (D != 64 && D != 128) || nc < 1) return 0;
+  return gdn2::scan_fwd_copies(n_bh, D, nc, in_place != 0);
+}
+
 int gdn2_debug_stream(int mode, const void* src, void* dst, size_t bytes, void* stream) {
   if (mode < 0 || mode > 2) return fail(GDN2_ERR_INVALID, "stream probe mode must be 0 (copy), 1 (read) or 2 (fill)");
   if (bytes == 0 || bytes % 4096) return fail(GDN2_ERR_INVALID, "stream probe bytes must be a positive multiple of 4096");

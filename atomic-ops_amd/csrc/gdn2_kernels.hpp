@@ -283,6 +283,7 @@ inline hipError_t persistent_grid(int n_chunks, dim3* grid) {
   return hipSuccess;
 }
 hipError_t launch_scan_fwd(int D, const ScanFwdArgs& a, hipStream_t s);
+int scan_fwd_copies(int n_bh, int D, int nc, bool in_place);
 hipError_t launch_out_fwd(int D, const OutFwdArgs& a, hipStream_t s);
 hipError_t launch_bwd_pre(int D, const BwdPreArgs& a, hipStream_t s);
 hipError_t launch_scan_bwd(int D, const ScanBwdArgs& a, hipStream_t s);

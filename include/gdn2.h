@@ -105,7 +105,8 @@ size_t gdn2_bwd_workspace_bytes(const gdn2_desc* d);
 
 /* Forward of one segment.  h0 may be NULL (zero state).  residual may be NULL for a
  * forward-only call (nothing is kept for a backward pass); otherwise it must hold
- * gdn2_residual_layout() bytes.  workspace holds gdn2_fwd_workspace_bytes(d, residual!=NULL). */
+ * gdn2_residual_layout() bytes.  workspace holds gdn2_fwd_workspace_bytes(d, residual!=NULL).
+ * h_final may be h0 (the state carried in place), here and in the other forwards below. */
 int gdn2_fwd(const gdn2_desc* d, const float* q, const float* k, const float* v, const float* w,
              const float* b, const float* g, const float* h0, float* o, float* h_final,
              void* residual, void* workspace, void* stream);
@@ -299,6 +300,10 @@ int gdn2_debug_stream(int mode, const void* src, void* dst, size_t bytes, void* 
  * out holds blocks * 256 floats; each is 512 * iters (the lane's accumulator sum for all-ones
  * operands).  1 <= blocks, iters <= 1 << 20. */
 int gdn2_debug_mfma(int blocks, int iters, float* out, void* stream);
+
+/* Diagnostics: the workgroups that run each 16-column slice's chain in the forward scan of n_bh
+ * (batch, head)s of nc 64-token chunks (in_place: h_final is h0); 0 on a bad shape. */
+int gdn2_debug_scan_copies(int n_bh, int D, int nc, int in_place);
 
 /* Per-kernel timing with HIP events recorded on the launch stream around every kernel.
  * gdn2_prof_begin(n) starts recording for up to n launches (process-wide, not re-entrant);

@@ -193,3 +193,14 @@ def prof_end():
     cnt = (_c_int * len(KERNEL_NAMES))()
     check(lib().gdn2_prof_end(ms, cnt), "gdn2_prof_end")
     return {n: (ms[i], cnt[i]) for i, n in enumerate(KERNEL_NAMES)}
+
+
+def restored(t, shape, dtype, device):
+    """A tensor that a node saved, as its backward kernel takes it.  Saved-tensor hooks may give back
+    anything (other dtypes, strides or devices, offloaded or compressed tensors); the kernels take
+    addresses, so the form is brought back here and another shape is refused."""
+    if t.shape != shape:
+        raise RuntimeError(f"saved-tensor hooks gave back shape {tuple(t.shape)} for a tensor of shape {tuple(shape)}")
+    if t.dtype != dtype or t.device != device:
+        t = t.to(device=device, dtype=dtype)
+    return t.contiguous()

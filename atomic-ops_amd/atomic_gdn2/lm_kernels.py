@@ -53,6 +53,16 @@ def _dense(t):
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
+def _save(ctx, *ts):
+    ctx.save_for_backward(*ts)
+    ctx.forms = [(t.shape, t.dtype, t.device) for t in ts]
+
+
+def _saved(ctx):
+    """The saved tensors in the form they were saved in."""
+    return tuple(_dense(_lib.restored(t, *f)) for t, f in zip(ctx.saved_tensors, ctx.forms))
+
+
 def _call(name, dev, *args):
     fn = getattr(_lib.lib(), name)
     with torch.cuda.device(dev):
@@ -210,7 +220,7 @@ class _PreMix(torch.autograd.Function):
         a = _PreMix._args(H, D, g_max, x, ps, y, outs, og)
         _call("gdn2_lm_premix_fwd", dev, ctypes.byref(a))
         ctx.dims = (H, D, g_max)
-        ctx.save_for_backward(x, *ps, wide, y, *outs, og)
+        _save(ctx, x, *ps, wide, y, *outs, og)
         return (*outs, og)
 
     @staticmethod
@@ -223,7 +233,7 @@ class _PreMix(torch.autograd.Function):
     @staticmethod
     def backward(ctx, *gs):
         H, D, g_max = ctx.dims
-        saved = ctx.saved_tensors
+        saved = _saved(ctx)
         x, ps, wide, y, outs, og = saved[0], saved[1:18], saved[18], saved[19], saved[20:26], saved[26]
         if torch.is_grad_enabled():
             return (None, None, None) + _vjp_through(_premix_ref(H, D, g_max), (x,) + ps, ctx.needs_input_grad[3:], gs)
@@ -254,12 +264,12 @@ class _PostMix(torch.autograd.Function):
     def forward(ctx, o, og, x, scale, wo):
         B, H, L, D = o.shape
         z = _rms(o, scale, og, (L, D))
-        ctx.save_for_backward(o, og, x, scale, wo, z)
+        _save(ctx, o, og, x, scale, wo, z)
         return torch.addmm(x.reshape(B * L, -1), z, wo).reshape(x.shape)
 
     @staticmethod
     def backward(ctx, dy):
-        o, og, x, scale, wo, z = ctx.saved_tensors
+        o, og, x, scale, wo, z = _saved(ctx)
         if torch.is_grad_enabled():
             return _vjp_through(_postmix_ref, (o, og, x, scale, wo), ctx.needs_input_grad, (dy,))
         need = ctx.needs_input_grad
@@ -282,12 +292,12 @@ class _Mlp(torch.autograd.Function):
         wide = _gather((wg, wu), 2 * wg.shape[1])
         gu = h @ wide
         act = _swiglu(gu)
-        ctx.save_for_backward(x, scale, wg, wu, wd, h, wide, gu, act)
+        _save(ctx, x, scale, wg, wu, wd, h, wide, gu, act)
         return torch.addmm(x2, act, wd).reshape(x.shape)
 
     @staticmethod
     def backward(ctx, dy):
-        x, scale, wg, wu, wd, h, wide, gu, act = ctx.saved_tensors
+        x, scale, wg, wu, wd, h, wide, gu, act = _saved(ctx)
         if torch.is_grad_enabled():
             return _vjp_through(_mlp_ref, (x, scale, wg, wu, wd), ctx.needs_input_grad, (dy,))
         need = ctx.needs_input_grad
@@ -302,12 +312,12 @@ class _Mlp(torch.autograd.Function):
 class _RmsNorm(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, scale):
-        ctx.save_for_backward(x, scale)
+        _save(ctx, x, scale)
         return _rms(x.reshape(-1, x.shape[-1]), scale).reshape(x.shape)
 
     @staticmethod
     def backward(ctx, dy):
-        x, scale = ctx.saved_tensors
+        x, scale = _saved(ctx)
         if torch.is_grad_enabled():
             return _vjp_through(rms_ref, (x, scale), ctx.needs_input_grad, (dy,))
         d2 = _dense(dy.reshape(-1, dy.shape[-1]))

@@ -139,16 +139,17 @@ def make_blr_trainable(cfg, scale, state_ckpt=None):
             if need_res:
                 ctx.save_for_backward(*xs, *res_list)
                 ctx.segs = segs
+                ctx.form, ctx.res_shapes = (xs[0].shape, dev), [r.shape for r in res_list]
                 ctx.dts = dts
             return o, h
 
         @staticmethod
         def backward(ctx, do, dhf):
-            saved = ctx.saved_tensors
-            xs, res_list = saved[:6], saved[6:]
+            saved, (shape, dev) = ctx.saved_tensors, ctx.form
+            xs = [_lib.restored(t, shape, torch.float32, dev) for t in saved[:6]]
+            res_list = [_lib.restored(t, n, torch.uint8, dev) for t, n in zip(saved[6:], ctx.res_shapes)]
             q = xs[0]
-            B, H, L, D = q.shape
-            dev = q.device
+            B, H, L, D = shape
             do = torch.zeros_like(q) if do is None else _f32(do)
             dh = q.new_zeros((B, H, D, D)) if dhf is None else _f32(dhf)
             grads = [torch.empty_like(q) for _ in range(6)]

@@ -95,6 +95,13 @@ struct Op {
   }
 };
 
+// A saved tensor as the backward takes it: saved-tensor hooks may give back other dtypes, strides or
+// devices (brought back here) or another shape (refused).
+Tensor restored(const Tensor& t, at::IntArrayRef size, at::ScalarType dt, const c10::Device& dev) {
+  TORCH_CHECK(t.defined() && t.sizes() == size, "saved-tensor hooks gave back another shape than was saved");
+  return t.to(dev, dt).contiguous();
+}
+
 // The whole call as one autograd node: forward and backward run the segment loop over views of the
 // full tensors (gdn2_desc.seq_ld), the state carried through h0 / h_final and dh0 / dh_final.
 // float32 inputs and clip <= 1e4 (then the reference's final cast of the gradients is the identity).
@@ -126,6 +133,8 @@ struct Sequence : torch::autograd::Function<Sequence> {
     ctx->save_for_backward(saved);
     ctx->saved_data["op"] = std::string(reinterpret_cast<const char*>(op), sizeof(Op));
     ctx->saved_data["h0"] = h0.has_value() && h0->requires_grad();
+    ctx->saved_data["shape"] = std::vector<int64_t>{B, H, L, D};
+    ctx->saved_data["device"] = q.device();
     return {o, h};
   }
 
@@ -134,10 +143,13 @@ struct Sequence : torch::autograd::Function<Sequence> {
     Op conf;
     std::memcpy(&conf, ctx->saved_data["op"].toStringRef().data(), sizeof(Op));
     const Op* op = &conf;
-    const Tensor* xs = saved.data();
-    const int64_t B = xs[0].size(0), H = xs[0].size(1), L = xs[0].size(2), D = xs[0].size(3);
-    c10::DeviceGuard guard(xs[0].device());
-    void* stream = stream_of(xs[0].device());
+    const std::vector<int64_t> shape = ctx->saved_data["shape"].toIntVector();
+    const int64_t B = shape[0], H = shape[1], L = shape[2], D = shape[3];
+    const c10::Device dev = ctx->saved_data["device"].toDevice();
+    c10::DeviceGuard guard(dev);
+    void* stream = stream_of(dev);
+    Tensor xs[6];
+    for (int i = 0; i < 6; ++i) xs[i] = restored(saved[i], shape, at::kFloat, dev);
     Tensor dout = gs[0].to(at::kFloat).contiguous(), dh = gs[1].to(at::kFloat).contiguous();
     Tensor gr[6];
     for (Tensor& t : gr) t = empty_on(xs[0], {B, H, L, D}, at::kFloat);
@@ -145,10 +157,13 @@ struct Sequence : torch::autograd::Function<Sequence> {
     for (int64_t s = n_seg - 1; s >= 0; --s) {
       const int64_t t0 = s * op->segment, x = t0 * D;
       const gdn2_desc d = op->training_desc(B, H, std::min(L - t0, op->segment), D, L);
+      size_t off[GDN2_RES_COUNT], total = 0;
+      TORCH_CHECK(abi.residual_layout(&d, off, &total) == 0, "gdn2_bwd: ", abi.last_error());
+      const Tensor res = restored(saved[6 + s], {(int64_t)total}, at::kByte, dev);
       Tensor ws = empty_on(xs[0], {(int64_t)abi.bwd_ws(&d)}, at::kByte);
       Tensor dh0 = empty_on(xs[0], {B, H, D, D}, at::kFloat);
       const int st = abi.bwd(&d, f32_at(xs[0], x), f32_at(xs[1], x), f32_at(xs[2], x), f32_at(xs[3], x),
-                             f32_at(xs[4], x), f32_at(xs[5], x), saved[6 + s].data_ptr(), f32_at(dout, x), f32_at(dh),
+                             f32_at(xs[4], x), f32_at(xs[5], x), res.data_ptr(), f32_at(dout, x), f32_at(dh),
                              f32_at(gr[0], x), f32_at(gr[1], x), f32_at(gr[2], x), f32_at(gr[3], x), f32_at(gr[4], x),
                              f32_at(gr[5], x), f32_at(dh0), ws.data_ptr(), stream);
       TORCH_CHECK(st == 0, "gdn2_bwd: ", abi.last_error());

@@ -85,3 +85,79 @@ def test_block_first_order_gradients_with_create_graph():
     kept = torch.autograd.grad(blk(x), leaves, w, create_graph=True)
     for a, b in zip(kept, plain):
         assert rel_l2(a.detach(), b) <= 2e-5
+
+
+def _hooks(pack):
+    return torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t)
+
+
+@pytest.mark.parametrize("pack", [lambda t: t.to(torch.bfloat16), lambda t: t.flip(0).flip(0).mT.contiguous().mT if t.dim() > 1 else t])
+def test_saved_tensors_in_another_form_reach_the_kernels_dense(cpu_passes, monkeypatch, pack):
+    """What saved-tensor hooks give back need not be what was saved: the backward kernels, which take
+    addresses, get dense float32 tensors of the saved shapes."""
+    K = cpu_passes
+    seen = []
+
+    def checked(*ts):
+        for t in ts:
+            assert t is None or (t.dtype == torch.float32 and t.is_contiguous())
+            seen.append(t)
+
+    def rms_bwd(x, scale, dy, gate=None, heads=None, res=None):
+        checked(x, scale, dy, gate, res)
+        return torch.zeros_like(x), torch.zeros_like(scale), None if gate is None else torch.zeros_like(gate)
+
+    def swiglu(gu, d_act=None):
+        checked(gu, d_act)
+        g, u = gu.chunk(2, dim=1)
+        return F.silu(g) * u if d_act is None else torch.zeros_like(gu)
+
+    monkeypatch.setattr(K, "_rms_bwd", rms_bwd)
+    monkeypatch.setattr(K, "_swiglu", swiglu)
+    monkeypatch.setattr(K, "_scatter", lambda wide, like: [torch.zeros_like(t) for t in like])
+    r = lambda *s: torch.randn(s).requires_grad_(True)  # noqa: E731
+    for node, xs in [(K._PostMix, [r(2, 2, 5, 4), r(10, 8), r(2, 5, 6), r(8), r(8, 6)]),
+                     (K._Mlp, [r(2, 5, 6), r(6), r(6, 8), r(6, 8), r(8, 6)]), (K._RmsNorm, [r(2, 5, 6), r(6)])]:
+        with _hooks(pack):
+            y = node.apply(*xs)
+        seen.clear()
+        torch.autograd.grad(y, xs, torch.ones_like(y))
+        assert len(seen) >= 3
+
+
+def test_saved_tensors_of_another_shape_are_refused(cpu_passes):
+    K = cpu_passes
+    xs = [torch.randn(2, 5, 6, requires_grad=True), torch.randn(6, requires_grad=True)]
+    with _hooks(lambda t: t[:1]):
+        y = K._RmsNorm.apply(*xs)
+    with pytest.raises(RuntimeError, match="saved-tensor hooks"):
+        torch.autograd.grad(y, xs, torch.ones_like(y))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("native", [True, False])
+def test_operator_with_saved_tensors_in_another_form(monkeypatch, native):
+    """The operator's node: inputs given back in bfloat16 (here bfloat16 values, so nothing is lost) are
+    widened, and a residual of another size is refused."""
+    if not torch.cuda.is_available():
+        pytest.skip("no ROCm GPU")
+    from atomic_gdn2 import make_blr_trainable
+    from test_bind import _python_only, _xs
+    from test_gpu_parity import base_cfg
+    if not native:
+        _python_only(monkeypatch)
+    fn = make_blr_trainable(base_cfg(max_chunks_per_call=1), 0.1)
+    xs = [x.bfloat16().float().requires_grad_(True) for x in _xs((1, 2, 128, 64))]
+
+    def grads(pack):
+        with _hooks(pack):
+            o, h = fn(*xs)
+        return torch.autograd.grad((o, h), xs, (o.detach(), h.detach()))
+
+    want = grads(lambda t: t)
+    for pack in (lambda t: t.bfloat16() if t.is_floating_point() else t,
+                 lambda t: t.mT.contiguous().mT if t.is_floating_point() else t):
+        assert all(torch.equal(a, b) for a, b in zip(grads(pack), want))
+    for pack in (lambda t: t if t.is_floating_point() else t[:-256], lambda t: t[:, :1] if t.is_floating_point() else t):
+        with pytest.raises(RuntimeError, match="saved-tensor hooks"):
+            grads(pack)

@@ -14,7 +14,8 @@ itself to be differentiated (``create_graph``) recomputes the step from ``_premi
 
 ``usable`` says where this path stands in for the module's own forward: float32 on the GPU, the
 block's own submodule types without hooks, the HIP operator as the mixer.  Everywhere else (the CPU,
-other dtypes, autocast, hooked, patched or replaced submodules, another mixer) the module forward runs.
+other dtypes, autocast, function transforms, forward mode, dispatch modes, tracing, hooked, patched or
+replaced submodules, another mixer) the module forward runs.
 """
 from __future__ import annotations
 
@@ -24,6 +25,8 @@ import weakref
 
 import torch
 import torch.nn.functional as F
+import torch.overrides
+import torch.utils._device
 
 from . import _lib
 
@@ -355,6 +358,20 @@ def _plain(m, cls):
             and not any(getattr(m, h) for h in _HOOKS))
 
 
+def _plain_mode():
+    """Whether a node of this module is an ordinary call here.  Function transforms and forward mode
+    have no rules for the nodes, and dispatch modes, function modes and tracers are to see the block's
+    operations; a default device (itself a function mode) is no reason."""
+    return not (torch.compiler.is_compiling()
+                or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch.autograd.forward_ad._current_level >= 0
+                or torch._C._len_torch_dispatch_stack() > 0
+                or torch._C._get_tracing_state() is not None
+                or (torch._C._len_torch_function_stack() > 0
+                    and any(type(m) is not torch.utils._device.DeviceContext
+                            for m in torch.overrides._get_current_function_mode_stack())))
+
+
 def _usable_input(x):
     return (x.is_cuda and type(x) in (torch.Tensor, torch.nn.Parameter) and _ready(x, x.device)
             and x.shape[-1] % 4 == 0 and x.shape[-1] <= _MAX_C and not torch.is_autocast_enabled("cuda")
@@ -380,7 +397,7 @@ def usable(block, x, dense, conv, norm):
     """Whether block_forward stands for block.forward(x); dense, conv, norm: the module types that
     the block is built of."""
     c = block.cfg
-    if operator_of(block.kernel_fn) is None or not (x.dim() == 3 and _usable_input(x)):
+    if operator_of(block.kernel_fn) is None or not (_plain_mode() and x.dim() == 3 and _usable_input(x)):
         return False
     if c.d_head not in (64, 128) or c.d_conv != 4 or c.proj_dim > _MAX_C or (c.mlp_mult * c.d_model) % 4:
         return False
@@ -407,7 +424,7 @@ def _tensors(m):
 
 
 def norm_usable(module, x, norm):
-    return (_plain(module, norm) and module.eps == _EPS and _usable_input(x)
+    return (_plain_mode() and _plain(module, norm) and module.eps == _EPS and _usable_input(x)
             and type(module.scale) in (torch.Tensor, torch.nn.Parameter) and module.scale.shape == x.shape[-1:]
             and _ready(module.scale, x.device))
 

@@ -254,7 +254,7 @@ def _prep_torch(g, seg, check_bad, B, H, L, D, bt):
     n_full, dev = L // bt, g.device
     L_full = n_full * bt
     flags = tflags = None
-    if seg is not None and n_full > 0:
+    if seg is not None and n_full > 0 and bt % 64 == 0:               # (the kernels refuse other chunks)
         first = seg[:, :L_full:bt]                                    # (B, n_full) id at each chunk start
         chg = torch.zeros_like(first, dtype=torch.bool)
         chg[:, 1:] = first[:, 1:] != first[:, :-1]
@@ -340,8 +340,9 @@ def chunk_forward_inference(q=None, k=None, v=None, w=None, b=None, g=None,
                 raise ValueError(f"{n} is on {t.device}, q on {dev}")
         xs, in_dtype = _inputs_for_kernel((q, k, v, w, b, g))
         xs[5] = _aligned(xs[5])
-    # (document ids of other integer or float types are formed by torch operations)
-    prep = _prep_native if runs and (seg is None or seg.dtype in _ID_TYPES) else _prep_torch
+    # (torch operations serve document ids of other integer or float types, and chunks that only the
+    # token kernel runs: prompts shorter than a chunk that is no multiple of 64)
+    prep = _prep_native if runs and bt % 64 == 0 and (seg is None or seg.dtype in _ID_TYPES) else _prep_torch
     flags, tflags, stats = prep(g if xs is None else xs[5], seg, check_bad, bsz, H, L, D, bt)
     o = h = None
     err = None

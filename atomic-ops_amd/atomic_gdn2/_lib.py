@@ -77,6 +77,7 @@ def lib():
         L.gdn2_fwd_bf16.argtypes = [P(Gdn2Desc)] + [_vp] * 12
         L.gdn2_fwd_noalloc.argtypes = [P(Gdn2Desc)] + [_vp] * 10
         L.gdn2_fwd_reset.argtypes = [P(Gdn2Desc), _c_int] + [_vp] * 12
+        L.gdn2_fwd_prefill.argtypes = [P(Gdn2Desc), _c_int] + [_vp] * 12
         L.gdn2_decode.argtypes = [P(Gdn2DecodeDesc)] + [_vp] * 13
         L.gdn2_prefill_prep.argtypes = [_c_int] * 6 + [_vp, _c_int] + [_vp] * 5
         L.gdn2_decode_flags.argtypes = [P(Gdn2DecodeDesc), _c_int] + [_vp] * 13
@@ -101,6 +102,7 @@ def lib():
         L.gdn2_prof_begin.argtypes = [_c_int]
         L.gdn2_prof_end.argtypes = [P(_c_dbl), P(_c_int)]
         for fn in ("gdn2_residual_layout", "gdn2_fwd", "gdn2_fwd_bf16", "gdn2_fwd_noalloc", "gdn2_fwd_reset",
+                   "gdn2_fwd_prefill",
                    "gdn2_decode", "gdn2_prefill_prep", "gdn2_decode_flags", "gdn2_bwd", "gdn2_wy_stage", "gdn2_scores", "gdn2_debug_gemm", "gdn2_debug_stream",
                    "gdn2_debug_mfma", "gdn2_lm_premix_fwd", "gdn2_lm_premix_bwd", "gdn2_lm_rms_fwd", "gdn2_lm_rms_bwd",
                    "gdn2_lm_swiglu", "gdn2_lm_columns", "gdn2_prof_begin", "gdn2_prof_end"):

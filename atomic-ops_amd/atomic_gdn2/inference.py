@@ -10,7 +10,7 @@ messages.  Tensors are torch tensors on a ROCm device and dtypes are torch dtype
 
 Kernels: ``decode_step`` and the prefill's tail (the tokens after its last full chunk) run the
 token-recurrence kernels (``gdn2_decode``); the prefill's full chunks run the residual-free
-forward with per-chunk state resets (``gdn2_fwd_reset``: the training forward's kernels, the
+forward with per-chunk state resets (``gdn2_fwd_prefill``: the training forward's kernels, the
 scan zeroing the state entering every chunk whose document differs from the previous chunk's).
 
 Two cases where the reference's code departs from its own documented contract ("a document
@@ -283,9 +283,9 @@ def _run_prefill(xs, in_dtype, cfg, scale, h, flags, tflags, sc, B, H, L, D):
         hf = torch.empty((B, H, D, D), dtype=torch.float32, device=dev)
         with torch.cuda.device(dev):
             ws = torch.empty(L_.gdn2_fwd_workspace_bytes(ctypes.byref(desc), 0), dtype=torch.uint8, device=dev)
-            _lib.check(L_.gdn2_fwd_reset(ctypes.byref(desc), in_dtype, *map(_lib.ptr, xs), _lib.ptr(h),
-                                         _lib.ptr(flags), _lib.ptr(o), _lib.ptr(hf), _lib.ptr(ws),
-                                         _lib.stream_handle(dev)), "gdn2_fwd_reset")
+            _lib.check(L_.gdn2_fwd_prefill(ctypes.byref(desc), in_dtype, *map(_lib.ptr, xs), _lib.ptr(h),
+                                           _lib.ptr(flags), _lib.ptr(o), _lib.ptr(hf), _lib.ptr(ws),
+                                           _lib.stream_handle(dev)), "gdn2_fwd_prefill")
         h = hf
     if L > L_full:
         st = None if h is None else h.to(_torch_dtype(sc)).contiguous()
@@ -325,8 +325,8 @@ def chunk_forward_inference(q=None, k=None, v=None, w=None, b=None, g=None,
     dev = q.device
     g_max_abs = float(cfg.g_max)
     # The domain of g and the document boundaries are checked on the device and read back in one
-    # synchronisation, while the prefill itself is already running: g is clamped to <= 0 (as on the
-    # decode path) only when some g > 0, and the kernels then run again.
+    # synchronisation, while the prefill itself is already running; its kernels clamp g to <= 0 as they
+    # load it.
     both = segment_ids is not None and cu_seqlens is not None
     check_bad = segment_ids is not None and n_full > 0
     if cu_seqlens is not None and not both:
@@ -352,7 +352,7 @@ def chunk_forward_inference(q=None, k=None, v=None, w=None, b=None, g=None,
             o, h = _run_prefill(xs, in_dtype, cfg, scale, hin, flags, tflags, sc, bsz, H, L, D)
         except (ValueError, _lib.Gdn2Error) as e:
             err = e                              # g's domain and the boundaries are reported first
-    lo, hi, has_bad = stats()
+    lo, _, has_bad = stats()
     # errors in the reference's order: g's domain, a boundary inside a chunk, both id forms
     if L > 0:
         # the layer's domain is [-g_max, 0] (NaN compares false, as in the reference)
@@ -376,9 +376,6 @@ def chunk_forward_inference(q=None, k=None, v=None, w=None, b=None, g=None,
         _check_device(q)
         if err is not None:
             raise err
-        if hi > 0:
-            xs[5] = torch.clamp(xs[5], max=0.0)
-            o, h = _run_prefill(xs, in_dtype, cfg, scale, hin, flags, tflags, sc, bsz, H, L, D)
     else:
         h = None if h0 is None else h0.to(torch.float32)
     if h is None:

@@ -219,11 +219,12 @@ int hip_fail(hipError_t e, const char* what) {
 // Fills it (anchor_kernel) from the raw gate g into buf; *anc = buf, or null when no piece is of
 // kind 2 or the pieces are formed exactly (nothing is launched then).
 int fill_anchors(const gdn2_desc* d, const gdn2::Cfg& cfg, const void* g, bool bf16, void* buf, hipStream_t s,
-                 const float** anc) {
+                 const float** anc, bool nonpos = false) {
   *anc = nullptr;
   // (the lean diagonal forms its kind-2 pieces exactly, without anchors)
   if (d->bs2 <= gdn2::T || d->diag == GDN2_DIAG_LEAN) return GDN2_OK;
-  gdn2::AnchorArgs aa{g, static_cast<float*>(buf), (int)((size_t)d->B * d->H * (d->L / gdn2::T)), d->bs2 / gdn2::T, cfg};
+  gdn2::AnchorArgs aa{g, static_cast<float*>(buf), (int)((size_t)d->B * d->H * (d->L / gdn2::T)), d->bs2 / gdn2::T, cfg,
+                      nonpos};
   const hipError_t e = timed(9, s, [&] { return gdn2::launch_anchors(d->D, aa, s, bf16); });
   if (e != hipSuccess) return hip_fail(e, "anchors launch");
   *anc = aa.anc;
@@ -291,10 +292,11 @@ size_t gdn2_bwd_workspace_bytes(const gdn2_desc* d) {
 
 namespace {
 // Forward of one segment; q..g are fp32 or (bf16 = true) bfloat16 bits.  reset: null, or (no
-// residual) one byte per (batch, head) and chunk, nonzero = zero state entering that chunk.
+// residual) one byte per (batch, head) and chunk, nonzero = zero state entering that chunk.  nonpos:
+// positive gates act as 0.
 int fwd_impl(const gdn2_desc* d, const void* q, const void* k, const void* v, const void* w, const void* b,
              const void* g, bool bf16, const float* h0, float* o, float* h_final, void* residual,
-             void* workspace, void* stream, const uint8_t* reset = nullptr) {
+             void* workspace, void* stream, const uint8_t* reset = nullptr, bool nonpos = false) {
   int st = residual ? validate_residual(d) : validate(d);
   if (st) return st;
   if (!q || !k || !v || !w || !b || !g || !o || !h_final || !workspace)
@@ -334,9 +336,10 @@ int fwd_impl(const gdn2_desc* d, const void* q, const void* k, const void* v, co
   }
 
   const float* anc = nullptr;
-  st = fill_anchors(d, cfg, g, bf16, anc_buf, s, &anc);
+  st = fill_anchors(d, cfg, g, bf16, anc_buf, s, &anc, nonpos);
   if (st) return st;
   gdn2::WyFwdArgs wa{};
+  if (nonpos) wa.g_top = 0.f;
   wa.q = q; wa.k = k; wa.v = v; wa.w = w; wa.b = b; wa.g = g; wa.anc = anc;
   wa.wp_f = wp; wa.uT_f = uT; wa.kg_f = kg; wa.qg_f = qg;
   wa.aqk_f = aqk; wa.A = A; wa.gl = gl;
@@ -440,6 +443,13 @@ int gdn2_fwd_reset(const gdn2_desc* d, int in_dtype, const void* q, const void* 
                    float* o, float* h_final, void* workspace, void* stream) {
   if (in_dtype != 0 && in_dtype != 1) return fail(GDN2_ERR_INVALID, "in_dtype must be 0 (fp32) or 1 (bf16)");
   return fwd_impl(d, q, k, v, w, b, g, in_dtype == 1, h0, o, h_final, nullptr, workspace, stream, chunk_reset);
+}
+
+int gdn2_fwd_prefill(const gdn2_desc* d, int in_dtype, const void* q, const void* k, const void* v,
+                     const void* w, const void* b, const void* g, const float* h0, const uint8_t* chunk_reset,
+                     float* o, float* h_final, void* workspace, void* stream) {
+  if (in_dtype != 0 && in_dtype != 1) return fail(GDN2_ERR_INVALID, "in_dtype must be 0 (fp32) or 1 (bf16)");
+  return fwd_impl(d, q, k, v, w, b, g, in_dtype == 1, h0, o, h_final, nullptr, workspace, stream, chunk_reset, true);
 }
 
 }  // extern "C"

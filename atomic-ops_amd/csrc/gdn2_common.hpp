@@ -517,19 +517,29 @@ __device__ __forceinline__ void wave_transpose16_n(float* tr, const float4* x, f
   }
 }
 
+__device__ __forceinline__ float4 min4(const float4& x, float top) {
+  return make_float4(__builtin_elementwise_minimum(x.x, top), __builtin_elementwise_minimum(x.y, top),
+                     __builtin_elementwise_minimum(x.z, top), __builtin_elementwise_minimum(x.w, top));
+}
+
 // In-chunk cumulative sum of g over the T rows of a (T x D) tile, into LDS sG (ld = LD).
 // Thread t owns float4 column t % (D/4) over a run of RUN consecutive rows: it sums its run,
 // then adds the totals of the runs above it in order.  Same code in every kernel, so every
 // kernel sees bit-identical gc.
 // LAST_READ: g is not read again by a later kernel (loaded with the non-temporal hint).
+// nonpos: positive gates act as 0.
 template <int D, int LD, int NTHREADS, bool LAST_READ = false, typename TIn>
-__device__ __forceinline__ void chunk_cumsum(const TIn* __restrict__ g, float* sG) {
+__device__ __forceinline__ void chunk_cumsum(const TIn* __restrict__ g, float* sG, bool nonpos = false) {
   constexpr int NQ = D / 4, NSEG = NTHREADS / NQ, RUN = T / NSEG;
   static_assert(NTHREADS % NQ == 0 && T % NSEG == 0 && RUN >= 1, "cumsum split");
   const int t = threadIdx.x, d = 4 * (t % NQ), s = t / NQ;
   float4 x[RUN];
 #pragma unroll
   for (int i = 0; i < RUN; ++i) x[i] = LAST_READ ? in_ldg4(g + (s * RUN + i) * D + d) : in_ld4(g + (s * RUN + i) * D + d);
+  if (nonpos) {
+#pragma unroll
+    for (int i = 0; i < RUN; ++i) x[i] = min4(x[i], 0.f);
+  }
 #pragma unroll
   for (int i = 1; i < RUN; ++i) x[i] = add4(x[i - 1], x[i]);
   st4(sG + (s * RUN + RUN - 1) * LD + d, x[RUN - 1]);
@@ -582,10 +592,13 @@ struct CumsumPass {
       }
     __syncthreads();
   }
-  __device__ __forceinline__ void run(float* sGf, float4* sTot) {
+  // gates above top act as top (+inf: none; a select would cost the hot kernels a branch)
+  __device__ __forceinline__ void run(float* sGf, float4* sTot, float top) {
 #pragma unroll
     for (int m = 0; m < NV; ++m)
       if (active(m)) {
+#pragma unroll
+        for (int i = 0; i < RUN; ++i) x[m][i] = min4(x[m][i], top);
 #pragma unroll
         for (int i = 1; i < RUN; ++i) x[m][i] = add4(x[m][i - 1], x[m][i]);
         sTot[seg(m) * NQP + col(m)] = x[m][RUN - 1];

@@ -378,7 +378,7 @@ __global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(NW ==
   for (int p = 0; p < NPASS; ++p) {
     // 1. gc = cumsum(g) inside the chunk, this pass's columns (fragment layout)
     if (a.g_is_gc) cs.store_as_is(sG);
-    else cs.run(sG, reinterpret_cast<float4*>(sQ));
+    else cs.run(sG, reinterpret_cast<float4*>(sQ), a.g_top);
 
     // 2. gated fragments (cd_slim.py:17-21): Kg = san(k e^{min(gl - gc, 0)}) as FRAG(Kg) (the
     //    forward scan turns its blocks around itself); Qg = san(q e^{min(gc, 0)}); X = b k e^{min(gc, 0)}
@@ -815,7 +815,7 @@ __global__ __launch_bounds__(512) void anchor_kernel(AnchorArgs a) {
   for (int j = 0; j < BMAX; ++j) {
     gl[j] = 0.f;
     if (j < B) {
-      chunk_cumsum<D, LD, 512>(static_cast<const TIn*>(a.g) + io_off<D>(a.cfg, blk * B + j), sG);
+      chunk_cumsum<D, LD, 512>(static_cast<const TIn*>(a.g) + io_off<D>(a.cfg, blk * B + j), sG, a.nonpos != 0);
       if (t < D) {
         if (j == 0) g00 = sG[t];
         gl[j] = sG[(T - 1) * LD + t];

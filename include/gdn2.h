@@ -137,6 +137,13 @@ int gdn2_fwd_reset(const gdn2_desc* d, int in_dtype, const void* q, const void* 
                    const uint8_t* chunk_reset, float* o, float* h_final, void* workspace,
                    void* stream);
 
+/* gdn2_fwd_reset with the positive entries of g acting as 0, as in gdn2_decode (the inference
+ * module's clamp, g <= 0), without a clamped copy of g. */
+int gdn2_fwd_prefill(const gdn2_desc* d, int in_dtype, const void* q, const void* k, const void* v,
+                     const void* w, const void* b, const void* g, const float* h0,
+                     const uint8_t* chunk_reset, float* o, float* h_final, void* workspace,
+                     void* stream);
+
 /* Token recurrence for serving (no MFMA; see gdn2_decode). */
 typedef struct gdn2_decode_desc {
   int32_t B, H, D;        /* D in {64, 128} */
@@ -168,12 +175,12 @@ int gdn2_decode(const gdn2_decode_desc* d, const void* q, const void* k, const v
                 const float* dt_bias, const uint8_t* reset, const void* state_in, void* o,
                 void* state_out, void* stream);
 
-/* Statistics and reset flags of a prefill, before gdn2_fwd_reset and gdn2_decode.  g (B,H,L,D) fp32
+/* Statistics and reset flags of a prefill, before gdn2_fwd_prefill and gdn2_decode.  g (B,H,L,D) fp32
  * (in_dtype 0) or bfloat16 bits (1), 16-byte aligned; seg NULL or B*L document ids, int32
  * (GDN2_FLAG_INT32) or int64 (GDN2_FLAG_INT64).  With n_full = L / bt full chunks:
  *   stats: GDN2_PREP_G_PARTS pairs (min, max of g over a part; NaN propagates), then, with seg,
  *     B*n_full floats: 1 when the chunk's ids are not all equal, else 0;
- *   flags (seg and n_full > 0): B*H*n_full*bt/64 bytes for gdn2_fwd_reset, set on a chunk whose
+ *   flags (seg and n_full > 0): B*H*n_full*bt/64 bytes for gdn2_fwd_prefill, set on a chunk whose
  *     first id differs from the previous chunk's;
  *   tail_flags (seg and L > n_full*bt): B*(L - n_full*bt) bytes for gdn2_decode, set on a token whose
  *     id differs from the previous token's. */

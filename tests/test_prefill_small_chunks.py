@@ -38,7 +38,7 @@ def test_longer_prompts_are_refused_in_order(docs):
     from atomic_gdn2.inference import chunk_forward_inference
     cfg, xs = _case(32, 80, 64)
     ids = torch.zeros(2, 80, dtype=torch.int64, device="cuda") if docs else None
-    with pytest.raises(ValueError, match="gdn2_fwd_reset"):
+    with pytest.raises(ValueError, match="gdn2_fwd_prefill"):
         chunk_forward_inference(*xs, 0.1, cfg, segment_ids=ids)
     xs[5][0, 0, 0, 0] = -100.0
     with pytest.raises(ValueError, match="outside the layer domain"):

@@ -138,6 +138,30 @@ def _weight_grad(x, dy):
     return halves[0] + halves[1]
 
 
+def _input_grad(dy, wide, width):
+    """dy wide^T, summed over one matrix's ``width`` columns at a time, as the products of the single
+    matrices are: rounding errors add up along a sum, and in one sum over all 4672 (2048) columns they
+    are 12.2e-7 (8.1e-7) of the result against 5.0e-7 (5.7e-7), which took the block's dx from 6.6e-7
+    of the exact one to 8.5e-7 (B4 L2048).  From 4096 rows on the parts accumulate into the result one
+    after the other (16384 rows: 536 -> 601 us, 237 -> 251); below, where launches cost more than
+    memory, they are one batched product and a sum (1280 rows: 55 -> 64 us, 28 -> 30).  For few rows
+    the library splits a single matrix's sum itself (256 rows: 2.6e-7, 2.9e-7; from 384 on it does
+    not), but not a batch's: quarters there (2.6e-7, 2.9e-7)."""
+    N, K = dy.shape
+    if N < 512:
+        width //= 4
+    m, d = K // width, wide.shape[0]
+    if N >= 4096:
+        dx = dy[:, :width] @ wide[:, :width].t()
+        for i in range(1, m):
+            a, b = i * width, (i + 1) * width if i + 1 < m else K
+            dx.addmm_(dy[:, a:b], wide[:, a:b].t())
+        return dx
+    p = torch.bmm(dy.as_strided((m, N, width), (width, K, 1)), wide.as_strided((m, width, d), (width, 1, K)))
+    dx = p[0] + p[1] if m == 2 else p.sum(0)
+    return dx if K == m * width else dx.addmm_(dy[:, m * width:], wide[:, m * width:].t())
+
+
 def _vjp_through(ref, inputs, needs, grads):
     """Gradients of ref(*inputs) for a backward that is itself differentiated.  They are taken at
     aliases of the inputs: an input may be computed from another one (the operator's o and the
@@ -251,7 +275,7 @@ class _PreMix(torch.autograd.Function):
         _call("gdn2_lm_premix_bwd", dev, ctypes.byref(a), (_vp * 6)(*(t.data_ptr() for t in ds[:6])), _addr(ds[6]),
               _addr(dy), _addr(dparam), _addr(ws))
         need = ctx.needs_input_grad[3:]
-        dx = (dy @ wide.t()).reshape(B, L, d) if need[0] else None
+        dx = _input_grad(dy, wide, C).reshape(B, L, d) if need[0] else None
         dws = _scatter(_weight_grad(x.reshape(N, d), dy), ps[:7]) if any(need[1:8]) else [None] * 7
         dps, o = [], 0
         for t in ps[7:]:
@@ -308,7 +332,7 @@ class _Mlp(torch.autograd.Function):
         dgu = _swiglu(gu, d2 @ wd.t())
         dwd = act.t() @ d2 if need[4] else None
         dwg, dwu = _scatter(h.t() @ dgu, (wg, wu)) if need[2] or need[3] else (None, None)
-        dx, dscale, _ = _rms_bwd(x.reshape(d2.shape), scale, dgu @ wide.t(), res=d2)
+        dx, dscale, _ = _rms_bwd(x.reshape(d2.shape), scale, _input_grad(dgu, wide, wg.shape[1]), res=d2)
         return tuple(g if n else None for g, n in zip((dx.reshape(x.shape), dscale, dwg, dwu, dwd), need))
 
 

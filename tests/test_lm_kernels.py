@@ -219,3 +219,21 @@ def test_a_patched_submodule_keeps_the_module_forward(monkeypatch):
             mp.setattr(cls, "forward", lambda self, y: 2.0 * f(self, y))
             assert not lm_kernels.usable(_block(cfg, op), x, *kinds)
             assert name != "mlp_norm" or not lm_kernels.norm_usable(_block(cfg, op).mlp_norm, x, e2e_lm.RMSNorm)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,L", [(1, 128), (1, 511), (1, 512), (2, 640), (1, 4095), (2, 2048)])   # quarters, parts, accumulated
+def test_input_gradients_as_exact_as_the_single_products(B, L):
+    """dx of the two nodes that multiply by several matrices at once, against float64: no further off
+    than the same in torch operations.  A norm over 65536 or more elements varies by well under 1 %;
+    5 % is left for the element-wise steps' own rounding (a sum over all columns at once is 40 % off,
+    or more)."""
+    _need_gpu()
+    from atomic_gdn2 import e2e_lm
+    cfg = e2e_lm.LMConfig()
+    for k in (0, 2):
+        ref, fused, xs = _passes(cfg, B, L, "cuda", torch.float32)[k]
+        exact = _run(ref, [x.detach().double().requires_grad_(True) for x in xs], 5)
+        at = len(exact) - len(xs)                       # the gradient of x
+        off = [rel_l2(_run(f, xs, 5)[at], exact[at]) for f in (fused, ref)]
+        assert off[0] <= 1.05 * off[1], (k, off)

@@ -129,13 +129,26 @@ def _scatter(wide, like):
 
 def _weight_grad(x, dy):
     """x^T dy over the rows, in two halves from 8192 rows on: the library's kernels for these shapes
-    leave one long reduction at 100 TFLOP/s, two batched halves run at 126 (16384 rows, 512 x 4672:
-    764 -> 620 us; 768 x 512: 122 -> 106 us; at 2048 rows the halves are slower, 98 against 91 us)."""
+    leave one long reduction at 100 TFLOP/s, two batched halves run at 126 (512 x 4672: 16384 rows
+    778 -> 614 us, 8192 378 -> 315, 4096 187 and 188; 768 x 512: 124 -> 105, 63 -> 59, 36 and 34).  The
+    MLP's products stay whole (512 x 2048: 16384 rows 254 and 246, 8192 126 and 124; 1024 x 512: 135 and
+    129, 67 and 70)."""
     n = x.shape[0]
     if n < 8192 or n % 2:
         return x.t() @ dy
     halves = torch.bmm(x.view(2, n // 2, -1).transpose(1, 2), dy.view(2, n // 2, -1))
     return halves[0] + halves[1]
+
+
+def _narrow_weight_grad(x, dy):
+    """x^T dy for a dy of a few columns.  The library splits such a product's long sum, which beside
+    the wide ones it does not (16384 rows, 512 x 6: 11.7e-7 of the result, as columns of the wide
+    product 15.7e-7 in halves, 22e-7 whole), but not over enough of the chip: 58 us.  Sixteen batched
+    parts from 4096 rows on: 3.0e-7, about 10 us."""
+    n = x.shape[0]
+    if n < 4096 or n % 16:
+        return x.t() @ dy
+    return torch.bmm(x.view(16, n // 16, -1).transpose(1, 2), dy.view(16, n // 16, -1)).sum(0)
 
 
 def _input_grad(dy, wide, width):
@@ -276,7 +289,11 @@ class _PreMix(torch.autograd.Function):
               _addr(dy), _addr(dparam), _addr(ws))
         need = ctx.needs_input_grad[3:]
         dx = _input_grad(dy, wide, C).reshape(B, L, d) if need[0] else None
-        dws = _scatter(_weight_grad(x.reshape(N, d), dy), ps[:7]) if any(need[1:8]) else [None] * 7
+        x2, dws = x.reshape(N, d), [None] * 7
+        if any(need[1:7]):
+            dws[:6] = _scatter(_weight_grad(x2, dy[:, :6 * C]), ps[:6])
+        if need[7]:
+            dws[6] = _narrow_weight_grad(x2, dy[:, 6 * C:6 * C + H])
         dps, o = [], 0
         for t in ps[7:]:
             dps.append(dparam[o:o + t.numel()].view(t.shape))

@@ -223,9 +223,9 @@ def test_a_patched_submodule_keeps_the_module_forward(monkeypatch):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,L", [(1, 128), (1, 511), (1, 512), (2, 640), (1, 4095), (2, 2048)])   # quarters, parts, accumulated
-def test_input_gradients_as_exact_as_the_single_products(B, L):
-    """dx of the two nodes that multiply by several matrices at once, against float64: no further off
-    than the same in torch operations.  A norm over 65536 or more elements varies by well under 1 %;
+def test_merged_products_as_exact_as_the_single_ones(B, L):
+    """dx of the two nodes that multiply by several matrices at once, and the gradient of the narrow
+    matrix among them, against float64: no further off than the same in torch operations.  A norm over 65536 or more elements varies by well under 1 %;
     5 % is left for the element-wise steps' own rounding (a sum over all columns at once is 40 % off,
     or more)."""
     _need_gpu()
@@ -235,5 +235,9 @@ def test_input_gradients_as_exact_as_the_single_products(B, L):
         ref, fused, xs = _passes(cfg, B, L, "cuda", torch.float32)[k]
         exact = _run(ref, [x.detach().double().requires_grad_(True) for x in xs], 5)
         at = len(exact) - len(xs)                       # the gradient of x
-        off = [rel_l2(_run(f, xs, 5)[at], exact[at]) for f in (fused, ref)]
+        got, want = _run(fused, xs, 5), _run(ref, xs, 5)
+        off = [rel_l2(y[at], exact[at]) for y in (got, want)]
         assert off[0] <= 1.05 * off[1], (k, off)
+        if k == 0:                                      # the decay projection's: 3072 elements, 10 %
+            off = [rel_l2(y[at + 7], exact[at + 7]) for y in (got, want)]
+            assert off[0] <= 1.1 * off[1], off

@@ -117,13 +117,10 @@ def _gather(parts, ld):
 
 
 def _scatter(wide, like):
-    """wide back into contiguous matrices of the shapes of ``like``."""
-    flat = torch.empty(sum(t.numel() for t in like), dtype=torch.float32, device=wide.device)
-    out, o = [], 0
-    for t in like:
-        out.append(flat[o:o + t.numel()].view(t.shape))
-        o += t.numel()
-    _columns(1, out, wide)
+    """wide back into matrices of the shapes of ``like`` (vectors from a wide of one row), each with a
+    storage of its own: they become parameters' gradients, which a program keeps, saves or frees singly."""
+    out = [torch.empty(t.shape, dtype=torch.float32, device=wide.device) for t in like]
+    _columns(1, [t.view(wide.shape[0], -1) for t in out], wide)
     return out
 
 
@@ -294,10 +291,7 @@ class _PreMix(torch.autograd.Function):
             dws[:6] = _scatter(_weight_grad(x2, dy[:, :6 * C]), ps[:6])
         if need[7]:
             dws[6] = _narrow_weight_grad(x2, dy[:, 6 * C:6 * C + H])
-        dps, o = [], 0
-        for t in ps[7:]:
-            dps.append(dparam[o:o + t.numel()].view(t.shape))
-            o += t.numel()
+        dps = _scatter(dparam.view(1, -1), ps[7:]) if any(need[8:]) else [None] * 10
         return (None, None, None) + tuple(g if n else None for g, n in zip([dx, *dws, *dps], need))
 
 

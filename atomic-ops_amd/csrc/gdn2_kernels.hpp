@@ -334,7 +334,7 @@ struct LmRmsArgs {
   int rows, C, L, D;
   float inv_c;
 };
-constexpr int LM_MAX_PARTS = 8;
+constexpr int LM_MAX_PARTS = 10;
 struct LmColumnsArgs {
   float* part[LM_MAX_PARTS];
   int width[LM_MAX_PARTS], start[LM_MAX_PARTS];

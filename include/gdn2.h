@@ -283,7 +283,7 @@ int gdn2_lm_rms_bwd(const gdn2_lm_rms* p, void* stream);
  * the gradient of gu for d_act (rows, M). */
 int gdn2_lm_swiglu(const float* gu, const float* d_act, float* out, int rows, int M, void* stream);
 
-/* n <= 8 matrices parts[j] (rows, widths[j]) and one (rows, ld) matrix that holds them side by side:
+/* n <= 10 matrices parts[j] (rows, widths[j]) and one (rows, ld) matrix that holds them side by side:
  * split 0 gathers them (columns past the last are zeroed), split 1 scatters it back.
  * rows <= 65535. */
 int gdn2_lm_columns(int split, float* const parts[], const int32_t widths[], int n, float* wide, int rows,

@@ -241,3 +241,16 @@ def test_merged_products_as_exact_as_the_single_ones(B, L):
         if k == 0:                                      # the decay projection's: 3072 elements, 10 %
             off = [rel_l2(y[at + 7], exact[at + 7]) for y in (got, want)]
             assert off[0] <= 1.1 * off[1], off
+
+
+@pytest.mark.gpu
+def test_gradients_have_storages_of_their_own():
+    _need_gpu()
+    from atomic_gdn2 import e2e_lm
+    cfg = e2e_lm.LMConfig(d_model=128, n_heads=3, d_head=64, n_layers=2)
+    model = e2e_lm.make_lm(cfg, seed=0)
+    e2e_lm.lm_loss(model, e2e_lm.synthetic_tokens(cfg, batch=2, length=128)).backward()
+    for n, p in model.named_parameters():
+        assert p.grad.shape == p.shape and p.grad.is_contiguous(), n
+        assert p.grad.untyped_storage().nbytes() == 4 * p.numel(), n
+    assert len({p.grad.data_ptr() for p in model.parameters()}) == len(list(model.parameters()))

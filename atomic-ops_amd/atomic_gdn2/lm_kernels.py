@@ -10,7 +10,8 @@ between the matrix products in one kernel each and the products that share an in
 
 Each is one autograd node whose backward runs the matching backward kernels.  A backward that is
 itself to be differentiated (``create_graph``) recomputes the step from ``_premix_ref`` /
-``_postmix_ref`` / ``_mlp_ref``, the same in torch operations.
+``_postmix_ref`` / ``_mlp_ref``, the same in torch operations; the operator between them is
+differentiable once, and a second derivative through it raises.
 
 ``usable`` says where this path stands in for the module's own forward: float32 on the GPU, the
 block's own submodule types without hooks, the HIP operator as the mixer.  Everywhere else (the CPU,

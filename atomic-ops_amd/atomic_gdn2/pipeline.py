@@ -7,7 +7,7 @@ Drop-in for the reference's ``atomic_gdn2/pipeline.py:17-66``:
 * sequences longer than ``cfg.max_chunks_per_call`` chunks are split into segments with the
   state carried through ``h0``/``h_final`` (pipeline.py:57-64);
 * the call is one custom autograd node (the analogue of the reference's per-segment
-  ``jax.custom_vjp``): its forward runs the HIP forward (``gdn2_fwd``) segment by segment and
+  ``jax.custom_vjp``), differentiable once: its forward runs the HIP forward (``gdn2_fwd``) segment by segment and
   keeps each segment's residual buffer, its backward runs ``gdn2_bwd`` over the segments in
   reverse and returns each segment's gradients through ``_fin`` (pipeline.py:11-14): sanitized
   at 1e4 and cast back to each input's dtype.  Segments are views into the full tensors
@@ -81,6 +81,19 @@ def _check_device(q):
     if q.device.type != "cuda":
         raise RuntimeError("atomic_gdn2 runs on the HIP kernels only: move the inputs to a ROCm "
                            f"device (got {q.device})")
+
+
+class _Once(torch.autograd.Function):
+    """The identity on n gradients of the operator, as functions of what they were formed from; raises
+    when they are differentiated."""
+
+    @staticmethod
+    def forward(ctx, n, *ts):
+        return tuple(t.view_as(t) for t in ts[:n])
+
+    @staticmethod
+    def backward(ctx, *gs):
+        raise RuntimeError("the GDN-2 operator is once differentiable: its gradients cannot be differentiated")
 
 
 def _segments(L, cfg):
@@ -166,7 +179,15 @@ def make_blr_trainable(cfg, scale, state_ckpt=None):
                     # cotangent of the previous segment's h_final (float32), or of the caller's h0
                     dh = dh0 if t0 == 0 else _fin(dh0, torch.float32, cfg)
             out = tuple(_fin(x, dt, cfg) for x, dt in zip(grads, ctx.dts[:6]))
-            return out + ((_fin(dh, ctx.dts[6], cfg),) if ctx.needs_input_grad[6] else (None,))
+            out = out + ((_fin(dh, ctx.dts[6], cfg),) if ctx.needs_input_grad[6] else (None,))
+            if torch.is_grad_enabled():
+                # a backward that keeps its graph: the kernels' gradients have no derivative, and say
+                # so when asked
+                n = 7 if ctx.needs_input_grad[6] else 6
+                # (casts and copies of the inputs have no history: a leaf of its own keeps the node in the graph)
+                leaf = torch.empty(0, requires_grad=True)
+                out = _Once.apply(n, *out[:n], *(t for t in (do, dhf) if t is not None), *saved[:6], leaf) + (None,) * (7 - n)
+            return out
 
     def forward_only(xs, h0):
         """No gradient needed: one kernel sequence over all L (no residual kept).  Equal bit for

@@ -102,6 +102,15 @@ Tensor restored(const Tensor& t, at::IntArrayRef size, at::ScalarType dt, const 
   return t.to(dev, dt).contiguous();
 }
 
+// The identity on the gradients of a Sequence, as functions of what they were formed from; raises when
+// they are differentiated.
+struct Once : torch::autograd::Function<Once> {
+  static variable_list forward(AutogradContext*, at::TensorList, const variable_list& grads) { return grads; }
+  static variable_list backward(AutogradContext*, variable_list) {
+    TORCH_CHECK(false, "the GDN-2 operator is once differentiable: its gradients cannot be differentiated");
+  }
+};
+
 // The whole call as one autograd node: forward and backward run the segment loop over views of the
 // full tensors (gdn2_desc.seq_ld), the state carried through h0 / h_final and dh0 / dh_final.
 // float32 inputs and clip <= 1e4 (then the reference's final cast of the gradients is the identity).
@@ -169,7 +178,19 @@ struct Sequence : torch::autograd::Function<Sequence> {
       TORCH_CHECK(st == 0, "gdn2_bwd: ", abi.last_error());
       dh = dh0;
     }
-    return {Tensor(), gr[0], gr[1], gr[2], gr[3], gr[4], gr[5], ctx->saved_data["h0"].toBool() ? dh : Tensor()};
+    variable_list out{gr[0], gr[1], gr[2], gr[3], gr[4], gr[5], ctx->saved_data["h0"].toBool() ? dh : Tensor()};
+    if (at::GradMode::is_enabled()) {
+      // a backward that keeps its graph: the kernels' gradients have no derivative, and say so when asked
+      if (!out.back().defined()) out.pop_back();
+      variable_list from(gs);
+      from.insert(from.end(), saved.begin(), saved.begin() + 6);
+      // (copies made of strided inputs have no history: a leaf of its own keeps the node in the graph)
+      from.push_back(at::empty({0}).requires_grad_(true));
+      out = Once::apply(at::TensorList(from), out);
+      out.resize(7);
+    }
+    out.insert(out.begin(), Tensor());
+    return out;
   }
 };
 

@@ -86,8 +86,10 @@ def lib():
         L.gdn2_scores.argtypes = [P(Gdn2Desc)] + [_vp] * 7
         L.gdn2_debug_gemm.argtypes = [_c_int, _vp, _vp, _vp, _c_int, _c_int, _c_int, _vp]
         L.gdn2_debug_stream.argtypes = [_c_int, _vp, _vp, _c_size, _vp]
-        L.gdn2_debug_scan_copies.argtypes = [_c_int] * 4
+        L.gdn2_debug_scan_copies.argtypes = [_c_int] * 5
         L.gdn2_debug_scan_copies.restype = _c_int
+        L.gdn2_debug_state_ckpt.argtypes = [P(Gdn2Desc), _c_int]
+        L.gdn2_debug_state_ckpt.restype = _c_int
         L.gdn2_debug_mfma.argtypes = [_c_int, _c_int, _vp, _vp]
         L.gdn2_lm_premix_workspace_bytes.argtypes = [_c_int] * 4
         L.gdn2_lm_premix_workspace_bytes.restype = _c_size

@@ -264,18 +264,19 @@ size_t gdn2_fwd_workspace_bytes(const gdn2_desc* d, int with_residual) {
 }
 
 // A checkpoint block's chunks run in sequence in bwd_state_rc, so K > 1 pays only when the blocks
-// fill the chip: D / 64 workgroups per chunk at K = 1, 512 resident at once (two per CU).  Up to one
-// and a half rounds every chunk is a block of its own; up to two, K = 2 fills exactly one round in the
-// same time with half the states kept.  Measured (bwd_state_rc, us, K = 1 / 2 / 3): B1 H2 L256
+// fill the chip: D / 64 workgroups per chunk at K = 1, two per CU resident at once (512 on 256 CUs).  Up
+// to one and a half rounds every chunk is a block of its own; up to two, K = 2 fills exactly one round in
+// the same time with half the states kept.  Measured (bwd_state_rc, us, K = 1 / 2 / 3): B1 H2 L256
 // 15 / 28 / 42; B4 H2 L2048 27 / 33 / 45; B4 H3 L2048 (768 workgroups at K = 1) 39 / 47 / 52;
 // B4 H4 L2048 (1024) 51 / 51 / 66; B4 H5 L2048 (1280) 59 / 72 / 69, the whole backward and forward
 // then equal at K = 1 and 3; B4 H6 L2048 69 / 73 / 70, where K = 3 saves 2 % of the whole step in the
 // forward's stores.
-int gdn2_default_state_ckpt(const gdn2_desc* d) {
+static int state_ckpt_rule(const gdn2_desc* d, int cus) {
   if (!d || d->B < 1 || d->H < 1 || d->L < 1) return 3;
   const int64_t wgs = (int64_t)d->B * d->H * (d->L / gdn2::T) * (d->D > 64 ? 2 : 1);
-  return wgs <= 768 ? 1 : wgs <= 1024 ? 2 : 3;
+  return wgs <= 3 * (int64_t)cus ? 1 : wgs <= 4 * (int64_t)cus ? 2 : 3;
 }
+int gdn2_default_state_ckpt(const gdn2_desc* d) { return state_ckpt_rule(d, gdn2::cu_count()); }
 
 // backward workspace: [dv_new | dh_next | dqg | dwp | dkg | dlast | X | Y | EZ (damped) |
 // anchors (bs2 > 64)]
@@ -758,10 +759,12 @@ int gdn2_lm_columns(int split, float* const parts[], const int32_t widths[], int
   return lm_done(gdn2::launch_lm_columns(a, split != 0, reinterpret_cast<hipStream_t>(stream)), "lm columns launch");
 }
 
-int gdn2_debug_scan_copies(int n_bh, int D, int nc, int in_place) {
+int gdn2_debug_scan_copies(int n_bh, int D, int nc, int in_place, int cus) {
   if (n_bh < 1 || (D != 64 && D != 128) || nc < 1) return 0;
-  return gdn2::scan_fwd_copies(n_bh, D, nc, in_place != 0);
+  return gdn2::scan_fwd_copies(n_bh, D, nc, in_place != 0, cus > 0 ? cus : gdn2::cu_count());
 }
+
+int gdn2_debug_state_ckpt(const gdn2_desc* d, int cus) { return state_ckpt_rule(d, cus > 0 ? cus : gdn2::cu_count()); }
 
 int gdn2_debug_stream(int mode, const void* src, void* dst, size_t bytes, void* stream) {
   if (mode < 0 || mode > 2) return fail(GDN2_ERR_INVALID, "stream probe mode must be 0 (copy), 1 (read) or 2 (fill)");

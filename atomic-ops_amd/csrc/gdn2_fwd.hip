@@ -851,13 +851,12 @@ hipError_t launch_anchors(int D, const AnchorArgs& a, hipStream_t s, bool bf16_i
   return hipGetLastError();
 }
 
-constexpr int WY_NW8_CHUNKS = 256;      // one chunk per CU (wy_fwd_kernel, NW)
-
 hipError_t launch_wy_fwd(int D, const WyFwdArgs& a, hipStream_t s, bool bf16_inputs) {
   // every piece has side min(bs2, 32) and, past bs2 = 64, kind 2
   const Piece& p0 = a.cfg.pieces.p[0];
   const int pm = p0.P < 16 ? PM_ELEM : a.cfg.diag == DIAG_LEAN ? PM_LEAN : p0.kind == 2 ? PM_WIDE : PM_TILES;
   if (pm == PM_WIDE && !a.anc) return hipErrorInvalidValue;
+  const bool eight_waves = a.n_chunks <= cu_count();      // at most one chunk per CU (wy_fwd_kernel, NW)
   dispatch_mode(a.cfg.dot_mode, [&](auto m) {
     constexpr int M = decltype(m)::value;
     auto go = [&](auto kern, int threads = 256) { hipLaunchKernelGGL(kern, dim3(a.n_chunks), dim3(threads), 0, s, a); };
@@ -867,7 +866,7 @@ hipError_t launch_wy_fwd(int D, const WyFwdArgs& a, hipStream_t s, bool bf16_inp
       if (pm == PM_ELEM) go(wy_fwd_kernel<DD, M, PM_ELEM, TI>);
       else if (pm == PM_LEAN) go(wy_fwd_kernel<DD, M, PM_LEAN, TI>);
       else if (pm == PM_WIDE) go(wy_fwd_kernel<DD, M, PM_WIDE, TI>);
-      else if (a.n_chunks <= WY_NW8_CHUNKS) go(wy_fwd_kernel<DD, M, PM_TILES, TI, 8>, 512);
+      else if (eight_waves) go(wy_fwd_kernel<DD, M, PM_TILES, TI, 8>, 512);
       else go(wy_fwd_kernel<DD, M, PM_TILES, TI>);
     };
     if (bf16_inputs) {

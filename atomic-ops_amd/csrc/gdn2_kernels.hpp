@@ -1,5 +1,7 @@
 // Kernel argument blocks and launch declarations shared by the HIP kernels and the C-ABI.
 #pragma once
+#include <atomic>
+
 #include "gdn2_common.hpp"
 
 namespace gdn2 {
@@ -275,6 +277,20 @@ hipError_t launch_anchors(int D, const AnchorArgs& a, hipStream_t s, bool bf16_i
 
 hipError_t launch_wy_fwd(int D, const WyFwdArgs& a, hipStream_t s, bool bf16_inputs = false);
 
+// CUs of the current device (a partition of a card has fewer than its 256; 256 without a device, for
+// rules asked on the host).
+inline int cu_count() {
+  static std::atomic<int> known[64];      // by device ordinal; 0: not asked yet
+  int dev = 0, ncu = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 256;
+  const bool keep = dev >= 0 && dev < 64;
+  if (keep) ncu = known[dev].load(std::memory_order_relaxed);
+  if (ncu > 0) return ncu;
+  if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 1) return 256;
+  if (keep) known[dev].store(ncu, std::memory_order_relaxed);
+  return ncu;
+}
+
 // Grid of a persistent kernel (one workgroup per CU, each walking chunks blockIdx.x,
 // + gridDim.x, ...): min(n_chunks, CUs of the current device).
 inline hipError_t persistent_grid(int n_chunks, dim3* grid) {
@@ -287,7 +303,7 @@ inline hipError_t persistent_grid(int n_chunks, dim3* grid) {
   return hipSuccess;
 }
 hipError_t launch_scan_fwd(int D, const ScanFwdArgs& a, hipStream_t s);
-int scan_fwd_copies(int n_bh, int D, int nc, bool in_place);
+int scan_fwd_copies(int n_bh, int D, int nc, bool in_place, int cus);
 hipError_t launch_out_fwd(int D, const OutFwdArgs& a, hipStream_t s);
 hipError_t launch_bwd_pre(int D, const BwdPreArgs& a, hipStream_t s);
 hipError_t launch_scan_bwd(int D, const ScanBwdArgs& a, hipStream_t s);

@@ -685,14 +685,14 @@ __global__ __launch_bounds__(8 * WAVE) void scan_bwd_kernel(ScanBwdArgs a) {
 // Copies of each slice while they still get a CU each (one workgroup fills a CU's registers).  One copy
 // where the state is carried in place (h_final is h0): copy 0 of a slice may finish before another one
 // has started and read its h0.
-int scan_fwd_copies(int n_bh, int D, int nc, bool in_place) {
-  const int r = 256 / (n_bh * (D / 16));
+int scan_fwd_copies(int n_bh, int D, int nc, bool in_place, int cus) {
+  const int r = cus / (n_bh * (D / 16));
   return in_place || r < 2 || nc < 2 ? 1 : r < 4 ? 2 : 4;
 }
 
 template <int D, int MODE>
 static void scan_fwd_launch(ScanFwdArgs a, hipStream_t s) {
-  a.copies = a.o ? scan_fwd_copies(a.n_bh, D, a.nc, a.h0 == a.hf) : 1;
+  a.copies = a.o ? scan_fwd_copies(a.n_bh, D, a.nc, a.h0 == a.hf, cu_count()) : 1;
   const dim3 grid(a.n_bh * (D / 16) * a.copies), block(512);
   if (!a.o) hipLaunchKernelGGL((scan_fwd_kernel<D, MODE, false, false>), grid, block, 0, s, a);
   else if (a.copies == 1) hipLaunchKernelGGL((scan_fwd_kernel<D, MODE, true, false>), grid, block, 0, s, a);

@@ -309,8 +309,10 @@ int gdn2_debug_stream(int mode, const void* src, void* dst, size_t bytes, void* 
 int gdn2_debug_mfma(int blocks, int iters, float* out, void* stream);
 
 /* Diagnostics: the workgroups that run each 16-column slice's chain in the forward scan of n_bh
- * (batch, head)s of nc 64-token chunks (in_place: h_final is h0); 0 on a bad shape. */
-int gdn2_debug_scan_copies(int n_bh, int D, int nc, int in_place);
+ * (batch, head)s of nc 64-token chunks (in_place: h_final is h0), 0 on a bad shape; and the interval
+ * of gdn2_default_state_ckpt.  Both for a device of cus CUs (0: the current one). */
+int gdn2_debug_scan_copies(int n_bh, int D, int nc, int in_place, int cus);
+int gdn2_debug_state_ckpt(const gdn2_desc* d, int cus);
 
 /* Per-kernel timing with HIP events recorded on the launch stream around every kernel.
  * gdn2_prof_begin(n) starts recording for up to n launches (process-wide, not re-entrant);

@@ -13,8 +13,8 @@ def test_one_workgroup_per_slice_in_place():
     from atomic_gdn2 import _lib
     copies = _lib.lib().gdn2_debug_scan_copies
     for n_bh, D, nc in [(1, 128, 2), (6, 128, 128), (16, 128, 9), (5, 64, 6), (32, 64, 2)]:
-        assert copies(n_bh, D, nc, 1) == 1 < copies(n_bh, D, nc, 0)
-    assert copies(0, 128, 4, 0) == copies(4, 96, 4, 0) == copies(4, 64, 0, 0) == 0
+        assert copies(n_bh, D, nc, 1, 256) == 1 < copies(n_bh, D, nc, 0, 256)
+    assert copies(0, 128, 4, 0, 256) == copies(4, 96, 4, 0, 256) == copies(4, 64, 0, 0, 256) == 0
 
 
 @pytest.mark.gpu

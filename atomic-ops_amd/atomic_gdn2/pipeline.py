@@ -37,18 +37,6 @@ def kernels_support(bt, wy_eps):
     return bt in SUPPORTED_BT and 0.0 <= wy_eps < 1.0
 
 
-# How the residual keeps the state for the backward (gdn2_desc.state_ckpt): K >= 1 keeps the
-# state entering the first chunk of each checkpoint block (blocks of K chunks; up to two chunks
-# left over become blocks of their own) and the backward recomputes the others inside its state
-# reductions; 0 keeps every chunk's (as the reference's residual does, pipeline.py:25).
-# The choice for state_ckpt=None is the library's (gdn2_default_state_ckpt): K = 3 for launches that
-# fill the chip, keeping 12 of every 32 states at or slightly below the stored form's time (MI355X,
-# B4 H6 D128: 0.4545 vs 0.4603 ms at L = 2048, 0.8807 vs 0.8945 ms at L = 4096; K = 4 keeps a
-# quarter for 3 % more time), and shorter blocks for smaller ones, whose backward is bound by a
-# block's length.
-DEFAULT_STATE_CKPT = 3
-
-
 def _fin(x, dt, cfg):
     """pipeline.py:11-14: pass through if already in dtype and clipped at <= 1e4."""
     if x.dtype == dt and cfg.clip <= _FINAL_CLIP:
@@ -103,10 +91,19 @@ def _segments(L, cfg):
     return [(t0, min(L, t0 + step)) for t0 in range(0, L, step)]
 
 
+# How the residual keeps the state for the backward (gdn2_desc.state_ckpt): K >= 1 keeps the
+# state entering the first chunk of each checkpoint block (blocks of K chunks; up to two chunks
+# left over become blocks of their own) and the backward recomputes the others inside its state
+# reductions; 0 keeps every chunk's (as the reference's residual does, pipeline.py:25).
+# The choice for state_ckpt=None is the library's (gdn2_default_state_ckpt): K = 3 for launches that
+# fill the chip, keeping 12 of every 32 states at or slightly below the stored form's time (MI355X,
+# B4 H6 D128: 0.4545 vs 0.4603 ms at L = 2048, 0.8807 vs 0.8945 ms at L = 4096; K = 4 keeps a
+# quarter for 3 % more time), and shorter blocks for smaller ones, whose backward is bound by a
+# block's length.
 def make_blr_trainable(cfg, scale, state_ckpt=None):
-    """``state_ckpt``: this build's residual knob (no counterpart in the reference), see
-    DEFAULT_STATE_CKPT; it changes memory and time, not results (the recomputed states equal
-    the stored ones bit for bit)."""
+    """``state_ckpt``: this build's residual knob (no counterpart in the reference): the interval K
+    above, None for the library's choice by shape; it changes memory and time, not results (the
+    recomputed states equal the stored ones bit for bit)."""
     scale = float(scale)
     ckpt = None if state_ckpt is None else int(state_ckpt)
     if ckpt is not None and ckpt < 0:

@@ -479,7 +479,7 @@ def main():
     ap.add_argument("--seed", type=int, default=0)
     ap.add_argument("--state-ckpt", type=int, default=None,
                     help="residual state checkpoint interval K (0 = every chunk's state kept); "
-                         "default: the library's DEFAULT_STATE_CKPT")
+                         "default: the library's choice for the shape")
     ap.add_argument("--ckpt-table", action="store_true", help="only print the state_ckpt table and exit")
     ap.add_argument("--dot-table", action="store_true", help="only print the dot-mode table and exit")
     ap.add_argument("--inference", action="store_true", help="only print the inference entry points' figures and exit")
@@ -527,8 +527,13 @@ def main():
     xs = [t.requires_grad_(True) for t in (q, k, v, w, b, g)]
     cfg = make_cfg(bt=64, bc=32, score_bs=64, bs2=32, mb=8, wy_eps=0.0, dot_mode="highest",
                    solve_dot_mode="highest", b3_dot_mode="highest")
-    from atomic_gdn2.pipeline import DEFAULT_STATE_CKPT
-    ckpt = DEFAULT_STATE_CKPT if args.state_ckpt is None else args.state_ckpt
+
+    def interval(L):
+        # the interval in use: the one asked for, or the library's for the workload at length L
+        seg = min(L, cfg.max_chunks_per_call * cfg.bt)
+        return _lib.training_desc(cfg, B_, H_, seg, D_, scale, L, args.state_ckpt).state_ckpt
+
+    ckpt = interval(L_)
     if args.ckpt_table:
         print(json.dumps({"state_ckpt_table": state_ckpt_table(cfg, args.seed)}), flush=True)
         return
@@ -550,15 +555,16 @@ def main():
         else:
             pts, pscale = make_inputs(B_, H_, args.seq_len, D_, seed=args.seed)
             pxs = [t.requires_grad_(True) for t in pts]
-        pfn = make_blr_trainable(cfg, pscale, state_ckpt=ckpt)
+        pfn = make_blr_trainable(cfg, pscale, state_ckpt=args.state_ckpt)
         for _ in range(args.warmup + args.steps):
             o, hf = pfn(*pxs)
             torch.autograd.grad((o, hf), pxs, grad_outputs=(2.0 * o, 2.0 * hf))
         torch.cuda.synchronize()
-        print(json.dumps({"profile_only": True, "B": B_, "H": H_, "L": args.seq_len, "state_ckpt": ckpt,
+        print(json.dumps({"profile_only": True, "B": B_, "H": H_, "L": args.seq_len,
+                          "state_ckpt": interval(args.seq_len),
                           "grad_evals": args.warmup + args.steps}), flush=True)
         return
-    fn = make_blr_trainable(cfg, scale, state_ckpt=ckpt)
+    fn = make_blr_trainable(cfg, scale, state_ckpt=args.state_ckpt)
 
     def step():
         # gradient of loss = sum(o^2) + sum(h_final^2): forward, the loss's cotangents

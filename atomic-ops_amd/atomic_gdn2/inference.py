@@ -331,13 +331,17 @@ def chunk_forward_inference(q=None, k=None, v=None, w=None, b=None, g=None,
     check_bad = segment_ids is not None and n_full > 0
     if cu_seqlens is not None and not both:
         segment_ids = _segment_ids_from_cu_seqlens(cu_seqlens, bsz, L, dev)
-    seg = None if segment_ids is None else torch.as_tensor(segment_ids, device=dev).reshape(bsz, L)
+    seg = None
+    if segment_ids is not None and (check_bad or not both):
+        seg = torch.as_tensor(segment_ids, device=dev).reshape(bsz, L)
+    # (an error of the run itself is kept: g's domain and the boundaries are reported first)
     runs = L > 0 and D in (64, 128) and dev.type == "cuda"
-    xs = None
+    xs = err = None
+    for t, n in zip((k, v, w, b, g), "kvwbg") if runs else ():
+        if t.device != dev:
+            runs, err = False, ValueError(f"{n} is on {t.device}, q on {dev}")
+            break
     if runs:
-        for t, n in zip((k, v, w, b, g), "kvwbg"):
-            if t.device != dev:
-                raise ValueError(f"{n} is on {t.device}, q on {dev}")
         xs, in_dtype = _inputs_for_kernel((q, k, v, w, b, g))
         xs[5] = _aligned(xs[5])
     # (torch operations serve document ids of other integer or float types, and chunks that only the
@@ -345,13 +349,12 @@ def chunk_forward_inference(q=None, k=None, v=None, w=None, b=None, g=None,
     prep = _prep_native if runs and bt % 64 == 0 and (seg is None or seg.dtype in _ID_TYPES) else _prep_torch
     flags, tflags, stats = prep(g if xs is None else xs[5], seg, check_bad, bsz, H, L, D, bt)
     o = h = None
-    err = None
     if runs and not both:
         hin = None if h0 is None else h0.to(torch.float32).to(dev).contiguous()
         try:
             o, h = _run_prefill(xs, in_dtype, cfg, scale, hin, flags, tflags, sc, bsz, H, L, D)
         except (ValueError, _lib.Gdn2Error) as e:
-            err = e                              # g's domain and the boundaries are reported first
+            err = e
     lo, _, has_bad = stats()
     # errors in the reference's order: g's domain, a boundary inside a chunk, both id forms
     if L > 0:

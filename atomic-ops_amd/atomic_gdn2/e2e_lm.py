@@ -148,8 +148,9 @@ class GDN2Block(nn.Module):
         self.down_proj = Dense(cfg.mlp_mult * d, d, False)
 
     def forward(self, x):
-        if lm_kernels.usable(self, x, Dense, CausalDepthwiseConv, RMSNorm):
-            return lm_kernels.block_forward(self, x)
+        ws = lm_kernels.block_tensors(self, x, Dense, CausalDepthwiseConv, RMSNorm)
+        if ws is not None:
+            return lm_kernels.block_forward(self, x, ws)
         cfg = self.cfg
         B, L, _ = x.shape
         H, D = cfg.n_heads, cfg.d_head

@@ -59,12 +59,16 @@ def _dense(t):
 
 def _save(ctx, *ts):
     ctx.save_for_backward(*ts)
-    ctx.forms = [(t.shape, t.dtype, t.device) for t in ts]
+    ctx.forms = _lib.bind().forms(ts)
 
 
 def _saved(ctx):
     """The saved tensors in the form they were saved in."""
-    return tuple(_dense(_lib.restored(t, *f)) for t, f in zip(ctx.saved_tensors, ctx.forms))
+    ts = ctx.saved_tensors
+    differ = _lib.bind().differ(ctx.forms, ts)
+    if not differ:
+        return ts
+    return tuple(t if f is None else _dense(_lib.restored(t, *f)) for t, f in zip(ts, differ))
 
 
 def _call(name, dev, *args):
@@ -432,22 +436,30 @@ def operator_of(mixer):
 def usable(block, x, dense, conv, norm):
     """Whether block_forward stands for block.forward(x); dense, conv, norm: the module types that
     the block is built of."""
+    return block_tensors(block, x, dense, conv, norm) is not None
+
+
+def block_tensors(block, x, dense, conv, norm):
+    """The block's weights as block_forward takes them, or None where the module forward runs."""
     c = block.cfg
     if operator_of(block.kernel_fn) is None or not (_plain_mode() and x.dim() == 3 and _usable_input(x)):
-        return False
+        return None
     if c.d_head not in (64, 128) or c.d_conv != 4 or c.proj_dim > _MAX_C or (c.mlp_mult * c.d_model) % 4:
-        return False
+        return None
     mods = block._modules
     if not (all(_plain(mods.get(n), dense) for n in _DENSE) and all(_plain(mods.get(n), conv) for n in _CONV)
             and all(_plain(mods.get(n), norm) and mods[n].eps == _EPS for n in _NORM)):
-        return False
+        return None
     if any((mods[n].bias is None) == (n in _BIASED) for n in _DENSE):
-        return False
+        return None
     d, p, H, M = c.d_model, c.proj_dim, c.n_heads, c.mlp_mult * c.d_model
     shapes = [(d, p)] * 6 + [(d, H)] + [(p, 4), (p,)] * 3 + [(p,)] * 2 + [(H,)] * 2 + [(p,), (p, d), (d,), (d, M), (d, M), (M, d)]
-    return x.shape[-1] == d and all(
-        type(t) in (torch.Tensor, torch.nn.Parameter) and t.shape == sh and _ready(t, x.device)
-        for t, sh in zip(_tensors(block), shapes))
+    if x.shape[-1] != d:
+        return None
+    ts = _tensors(block)
+    if not all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.shape == sh for t, sh in zip(ts, shapes)):
+        return None
+    return ts if _lib.bind().dense(ts, x) else None
 
 
 def _tensors(m):
@@ -469,8 +481,8 @@ def rms_norm(module, x):
     return _RmsNorm.apply(x, module.scale)
 
 
-def block_forward(m, x):
-    c, ws = m.cfg, _tensors(m)
+def block_forward(m, x, ws):
+    c = m.cfg
     *ops, og = _PreMix.apply(c.n_heads, c.d_head, c.g_max, x, *ws[:17])
     o, _ = operator_of(m.kernel_fn)(*ops)
     x = _PostMix.apply(o, og, x, *ws[17:19])

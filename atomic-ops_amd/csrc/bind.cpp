@@ -14,11 +14,14 @@
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
+#include <torch/csrc/Device.h>
+#include <torch/csrc/DynamicTypes.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstring>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -380,10 +383,99 @@ PyObject* py_decode(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// What a saved tensor looked like (lm_kernels.py): forty of them a block, looked over in Python at 1.5 us
+// each, would be a fifth of a small block's host time.
+struct Form {
+  std::vector<int64_t> sizes;
+  at::ScalarType dtype;
+  c10::Device device;
+};
+const char* const kFormsName = "atomic_gdn2._bind.forms";
+void free_forms(PyObject* cap) { delete static_cast<std::vector<Form>*>(PyCapsule_GetPointer(cap, kFormsName)); }
+bool tensors_of(PyObject* t) {
+  if (!PyTuple_Check(t)) return false;
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(t); ++i)
+    if (!THPVariable_Check(PyTuple_GET_ITEM(t, i))) return false;
+  return true;
+}
+
+// forms(tensors): their sizes, dtypes and devices
+PyObject* py_forms(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 1 || !tensors_of(args[0])) return PyErr_Format(PyExc_TypeError, "forms takes a tuple of tensors");
+  auto f = std::make_unique<std::vector<Form>>();
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(args[0]); ++i) {
+    const Tensor& t = THPVariable_Unpack(PyTuple_GET_ITEM(args[0], i));
+    f->push_back(Form{t.sizes().vec(), t.scalar_type(), t.device()});
+  }
+  PyObject* cap = PyCapsule_New(f.get(), kFormsName, free_forms);
+  if (cap) f.release();
+  return cap;
+  END_HANDLE_TH_ERRORS
+}
+
+// differ(forms, tensors) -> None when every tensor has its form, contiguous and 16-byte aligned; else
+// a list with (sizes, dtype, device) for those that do not, None for the others
+PyObject* py_differ(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 2 || !tensors_of(args[1])) return PyErr_Format(PyExc_TypeError, "differ takes forms and a tuple of tensors");
+  const auto* f = static_cast<const std::vector<Form>*>(PyCapsule_GetPointer(args[0], kFormsName));
+  if (!f) return nullptr;
+  if ((Py_ssize_t)f->size() != PyTuple_GET_SIZE(args[1])) return PyErr_Format(PyExc_ValueError, "another number of tensors");
+  auto same = [&](const Tensor& t, const Form& o) {
+    return t.layout() == c10::kStrided && t.sizes() == at::IntArrayRef(o.sizes) && t.scalar_type() == o.dtype &&
+           t.device() == o.device && t.is_contiguous() && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
+  };
+  bool all = true;
+  for (size_t i = 0; i < f->size() && all; ++i) all = same(THPVariable_Unpack(PyTuple_GET_ITEM(args[1], i)), (*f)[i]);
+  if (all) return none();
+  PyObject* out = PyList_New((Py_ssize_t)f->size());
+  for (size_t i = 0; out && i < f->size(); ++i) {
+    const Form& o = (*f)[i];
+    PyObject* x = Py_None;
+    if (same(THPVariable_Unpack(PyTuple_GET_ITEM(args[1], i)), o)) {
+      Py_INCREF(x);
+    } else {
+      PyObject *sz = PyTuple_New((Py_ssize_t)o.sizes.size()), *dev = THPDevice_New(o.device);
+      for (size_t k = 0; sz && k < o.sizes.size(); ++k) PyTuple_SET_ITEM(sz, (Py_ssize_t)k, PyLong_FromLongLong(o.sizes[k]));
+      PyObject* dt = reinterpret_cast<PyObject*>(torch::getTHPDtype(o.dtype));
+      x = sz && dev ? PyTuple_Pack(3, sz, dt, dev) : nullptr;
+      Py_XDECREF(sz);
+      Py_XDECREF(dev);
+      if (!x) {
+        Py_DECREF(out);
+        return nullptr;
+      }
+    }
+    PyList_SET_ITEM(out, (Py_ssize_t)i, x);
+  }
+  return out;
+  END_HANDLE_TH_ERRORS
+}
+
+// dense(tensors, x) -> whether each is as the kernels read it: float32, on x's device, contiguous,
+// 16-byte aligned, not empty
+PyObject* py_dense(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 2 || !tensors_of(args[0]) || !THPVariable_Check(args[1])) return PyErr_Format(PyExc_TypeError, "dense takes a tuple of tensors and a tensor");
+  const c10::Device dev = THPVariable_Unpack(args[1]).device();
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(args[0]); ++i) {
+    const Tensor& t = THPVariable_Unpack(PyTuple_GET_ITEM(args[0], i));
+    if (t.layout() != c10::kStrided || t.device() != dev || t.scalar_type() != at::kFloat || t.numel() == 0 || !t.is_contiguous() ||
+        (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) != 0)
+      Py_RETURN_FALSE;
+  }
+  Py_RETURN_TRUE;
+  END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef methods[] = {
     {"bind", (PyCFunction)(void (*)())py_bind, METH_FASTCALL, "bind(*addresses)"},
     {"op", (PyCFunction)(void (*)())py_op, METH_FASTCALL, "op(desc, segment)"},
     {"sequence", (PyCFunction)(void (*)())py_sequence, METH_FASTCALL, "sequence(op, q, k, v, w, b, g, h0)"},
+    {"forms", (PyCFunction)(void (*)())py_forms, METH_FASTCALL, "forms(tensors)"},
+    {"differ", (PyCFunction)(void (*)())py_differ, METH_FASTCALL, "differ(forms, tensors)"},
+    {"dense", (PyCFunction)(void (*)())py_dense, METH_FASTCALL, "dense(tensors, x)"},
     {"decode", (PyCFunction)(void (*)())py_decode, METH_FASTCALL, "decode(...)"},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module{PyModuleDef_HEAD_INIT, "_bind", "native call path of the operator", -1, methods};

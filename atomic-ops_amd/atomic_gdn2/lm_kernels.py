@@ -153,28 +153,25 @@ def _narrow_weight_grad(x, dy):
     return torch.bmm(x.view(16, n // 16, -1).transpose(1, 2), dy.view(16, n // 16, -1)).sum(0)
 
 
-def _input_grad(dy, wide, width):
-    """dy wide^T, summed over one matrix's ``width`` columns at a time, as the products of the single
-    matrices are: rounding errors add up along a sum, and in one sum over all 4672 (2048) columns they
-    are 12.2e-7 (8.1e-7) of the result against 5.0e-7 (5.7e-7), which took the block's dx from 6.6e-7
-    of the exact one to 8.5e-7 (B4 L2048).  From 4096 rows on the parts accumulate into the result one
-    after the other (16384 rows: 536 -> 601 us, 237 -> 251); below, where launches cost more than
-    memory, they are one batched product and a sum (1280 rows: 55 -> 64 us, 28 -> 30).  For few rows
-    the library splits a single matrix's sum itself (256 rows: 2.6e-7, 2.9e-7; from 384 on it does
-    not), but not a batch's: quarters there (2.6e-7, 2.9e-7)."""
+def _input_grad(dy, wide, parts, parts_few):
+    """dy wide^T with the sum over the columns in parts.  Rounding errors add up along a sum: as whole
+    sums over 4672 and 2048 columns (12.2e-7 and 8.1e-7 of the result) these two products took the
+    block's dx from 6.6e-7 of the exact one, where a product per matrix has it, to 8.5e-7 (B4 L2048).
+    Halves of the one and quarters of the other (8.6e-7, 4.1e-7; the MLP's weighs more in dx) keep it at
+    6.5e-7, in less time than one part per matrix (601 + 251 us at 16384 rows, 253 + 103 at 4864):
+    from 8192 rows on the parts accumulate into the result one after the other (16384 rows: 525 ->
+    539 us and 237 -> 273), below they are one batched product and a sum (4864: 200 -> 193 and
+    89 -> 99).  For few rows the library splits a single matrix's sum by itself (up to 256 rows:
+    2.6e-7, 2.9e-7), but not a batch's: parts_few below 512."""
     N, K = dy.shape
-    if N < 512:
-        width //= 4
-    m, d = K // width, wide.shape[0]
-    if N >= 4096:
-        dx = dy[:, :width] @ wide[:, :width].t()
-        for i in range(1, m):
-            a, b = i * width, (i + 1) * width if i + 1 < m else K
-            dx.addmm_(dy[:, a:b], wide[:, a:b].t())
+    m = parts if N >= 512 else parts_few
+    w = K // m
+    if N >= 8192:
+        dx = dy[:, :w] @ wide[:, :w].t()
+        for i in range(w, K, w):
+            dx.addmm_(dy[:, i:i + w], wide[:, i:i + w].t())
         return dx
-    p = torch.bmm(dy.as_strided((m, N, width), (width, K, 1)), wide.as_strided((m, width, d), (width, 1, K)))
-    dx = p[0] + p[1] if m == 2 else p.sum(0)
-    return dx if K == m * width else dx.addmm_(dy[:, m * width:], wide[:, m * width:].t())
+    return torch.bmm(dy.view(N, m, w).transpose(0, 1), wide.view(-1, m, w).permute(1, 2, 0)).sum(0)
 
 
 def _vjp_through(ref, inputs, needs, grads):
@@ -290,7 +287,7 @@ class _PreMix(torch.autograd.Function):
         _call("gdn2_lm_premix_bwd", dev, ctypes.byref(a), (_vp * 6)(*(t.data_ptr() for t in ds[:6])), _addr(ds[6]),
               _addr(dy), _addr(dparam), _addr(ws))
         need = ctx.needs_input_grad[3:]
-        dx = _input_grad(dy, wide, C).reshape(B, L, d) if need[0] else None
+        dx = _input_grad(dy, wide, 2, 32).reshape(B, L, d) if need[0] else None
         x2, dws = x.reshape(N, d), [None] * 7
         if any(need[1:7]):
             dws[:6] = _scatter(_weight_grad(x2, dy[:, :6 * C]), ps[:6])
@@ -348,7 +345,7 @@ class _Mlp(torch.autograd.Function):
         dgu = _swiglu(gu, d2 @ wd.t())
         dwd = act.t() @ d2 if need[4] else None
         dwg, dwu = _scatter(h.t() @ dgu, (wg, wu)) if need[2] or need[3] else (None, None)
-        dx, dscale, _ = _rms_bwd(x.reshape(d2.shape), scale, _input_grad(dgu, wide, wg.shape[1]), res=d2)
+        dx, dscale, _ = _rms_bwd(x.reshape(d2.shape), scale, _input_grad(dgu, wide, 4, 8), res=d2)
         return tuple(g if n else None for g, n in zip((dx.reshape(x.shape), dscale, dwg, dwu, dwd), need))
 
 

@@ -108,10 +108,10 @@ def _swiglu(gu, d_act=None):
 
 
 def _columns(split, parts, wide):
-    n = len(parts)
+    n, rows = len(parts), wide.shape[0]
     ptrs = (_vp * n)(*(t.data_ptr() for t in parts))
-    widths = (_i32 * n)(*(t.shape[1] for t in parts))
-    _call("gdn2_lm_columns", wide.device, int(split), ptrs, widths, n, _addr(wide), wide.shape[0], wide.shape[1])
+    widths = (_i32 * n)(*(t.numel() // rows for t in parts))
+    _call("gdn2_lm_columns", wide.device, int(split), ptrs, widths, n, _addr(wide), rows, wide.shape[1])
 
 
 def _gather(parts, ld):
@@ -125,7 +125,7 @@ def _scatter(wide, like):
     """wide back into matrices of the shapes of ``like`` (vectors from a wide of one row), each with a
     storage of its own: they become parameters' gradients, which a program keeps, saves or frees singly."""
     out = [torch.empty(t.shape, dtype=torch.float32, device=wide.device) for t in like]
-    _columns(1, [t.view(wide.shape[0], -1) for t in out], wide)
+    _columns(1, out, wide)
     return out
 
 

@@ -14,8 +14,8 @@
 // Element-wise, no MFMA: 2 D^2 state elements per (batch, head), plus 7 D per token.
 //   one token (decode_step_kernel): memory-bound at serving batches, so a wave reads whole lines:
 //     thread t owns 4 columns (j0 = 4 (t % (CW/4))) of the D/16 key rows of group t / (CW/4); the key
-//     vectors go through LDS and the key sums over the 16 groups too.  B64 H16 D128 fp32: 27.5 us,
-//     0.79 of the copy rate.
+//     vectors go through LDS and the key sums over the 16 groups too.  B64 H16 D128 fp32: 26.6 us,
+//     0.81 of the copy rate.
 //   several tokens (decode_tail_kernel): bound by a token's dependent chain, so nothing on it goes
 //     through memory or a barrier: a lane holds 4 columns of 4 key rows, a key sum is 4 products per
 //     lane and a butterfly over the D/4 lanes of its columns, and the next tokens' operands are loaded

@@ -14,7 +14,7 @@
 // stored ones, and leave per-workgroup partial sums of the parameter gradients that lm_reduce adds
 // in a fixed order.
 // The benchmark LM's forward and backward (B8 L2048, 8 blocks): 73.5 ms with torch's passes, of
-// which about 33 were these chains, 39.6 ms with the kernels below (3.8 ms of them).
+// which about 33 were these chains, 38.4 ms with the kernels below (4.5 ms of them).
 #include "gdn2_kernels.hpp"
 
 namespace gdn2 {

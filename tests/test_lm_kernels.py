@@ -106,7 +106,8 @@ def test_saturated_and_non_finite_rows():
 @pytest.mark.gpu
 def test_block_is_the_module_forward():
     """The whole block through the HIP passes against the module's own forward (same operator), values
-    and all gradients; a backward to be differentiated again goes through torch operations."""
+    and all gradients; and the RMS norm's backward that is differentiated again (the other nodes':
+    test_lm_autograd.py)."""
     _need_gpu()
     from atomic_gdn2 import e2e_lm, lm_kernels
     cfg = e2e_lm.LMConfig(d_model=128, n_heads=3, d_head=64)
